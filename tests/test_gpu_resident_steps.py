@@ -343,6 +343,69 @@ def test_attention_ignores_rows_past_the_range(env, heads, kv_heads, width, leng
         dev.close()
 
 
+RUN_CASES = [  # heads, kv_heads, width, max_length, count, first, window: count * heads past the tile kernel's threshold
+    (32, 8, 128, 300, 64, 0, 0), (32, 8, 128, 700, 70, 601, 0), (32, 4, 64, 129, 65, 64, 0), (24, 8, 128, 250, 100, 33, 0),
+    (32, 32, 128, 97, 97, 0, 40), (32, 1, 64, 200, 64, 130, 0), (32, 8, 128, 600, 513, 40, 64), (16, 8, 256, 300, 257, 17, 0),
+    (16, 8, 256, 400, 256, 140, 100), (8, 2, 128, 8300, 257, 8000, 0), (64, 8, 256, 600, 512, 80, 0)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,width,max_length,count,first,window", RUN_CASES,
+                         ids=[f"{h}/{k}x{w}-q{c}-p{f}-w{win}" for h, k, w, n, c, f, win in RUN_CASES])
+@pytest.mark.parametrize("form", ["run", "any-order"])
+def test_attention_runs(env, heads, kv_heads, width, max_length, count, first, window, form):
+    """Runs long enough for the matrix-core kernel: ragged row tiles, head
+    groups that do not divide a tile, ranges that start and end inside key
+    tiles. any-order: the positions in no order, one token without a range
+    (its output is left alone), and NaN and infinities in every cached row
+    that some tokens see and others do not: the tokens that see one give a
+    non-finite output, every other token is as if the row were not there."""
+    rt, L, stream = env
+    rng = np.random.default_rng(max_length * 5 + width + count)
+    q_stride = (heads + 2 * kv_heads) * width
+    q = rng.standard_normal((count, q_stride)).astype(np.float32)
+    keys = rng.standard_normal((max_length, kv_heads * width)).astype(np.float32)
+    values = rng.standard_normal((max_length, kv_heads * width)).astype(np.float32)
+    positions = np.arange(first, first + count, dtype=np.int32)
+    keys[first + count:], values[first + count:] = np.nan, np.inf
+    poison = []
+    if form == "any-order":
+        rng.shuffle(positions)
+        positions[count // 3] = -1
+        poison = [first + count // 2, first + count - 2]
+        values[poison[0], ::3] = np.inf
+        keys[poison[1], 5::7] = np.nan
+        values[poison[1], 1::2] = np.nan
+    scale = float(1 / np.sqrt(np.float32(width)))
+    sees = [p >= 0 and any(t <= p and (not window or t > p - window) for t in poison) for p in positions]
+    check = [i for i in range(count) if positions[i] >= 0 and not sees[i]]
+    check = check if len(check) <= 70 else check[:24] + check[-24:] + list(rng.choice(check[24:-24], 22, replace=False))
+    dev = Dev(rt)
+    try:
+        qd, kd, vd, pd = dev.put(q), dev.put(keys), dev.put(values), dev.put(positions)
+        od = dev.put(np.full((count, heads * width), 7.0, np.float32))
+        sd = dev.empty(4 * count * heads * max_length) if max_length > 8192 else 0
+        print(f"attention run {heads}/{kv_heads} x {width}, {count} from {first}, window {window}, {form}", flush=True)
+        assert L.nya_hip_attention(qd, q_stride, kd, vd, od, sd, pd, count, heads, kv_heads, width, max_length,
+                                   window, scale, stream) == 0
+        rt.sync(stream)
+        got = dev.get(od, np.empty((count, heads * width), np.float32))
+    finally:
+        dev.close()
+    worst = 0.0
+    for i in check:
+        ref = attention_ref(q[i, :heads * width], keys, values, heads, kv_heads, width, int(positions[i]) + 1,
+                            np.float32(scale), window)
+        worst = max(worst, scaled_error(got[i], ref))
+    print(f"  scaled error {worst:.3g} over {len(check)} tokens", flush=True)
+    assert worst <= 2e-6   # fp32 sums and products over unit-variance values (the per-head kernel: 1e-6)
+    for i in range(count):
+        if positions[i] < 0:
+            assert np.all(got[i] == 7.0)
+        else:
+            # A seen NaN key (any head) or infinite value leaves no row clean.
+            assert np.all(np.isfinite(got[i])) != sees[i]
+
+
 SPLIT_CASES = [(32, 8, 128, 4096, 1, 64, 0), (32, 4, 64, 1000, 1, 16, 0), (8, 8, 128, 300, 1, 8, 0),
                (16, 8, 128, 2000, 3, 32, 0), (8, 2, 256, 5000, 2, 8, 0), (32, 4, 64, 20000, 1, 32, 0),
                (32, 8, 128, 5, 1, 64, 0), (32, 8, 128, 257, 33, 8, 0), (8, 2, 128, 600, 2, 300, 0),
