@@ -94,8 +94,8 @@ hipError_t launch_smalln_rows(unsigned type, const uint8_t *w, const float *x, f
 hipError_t launch_quantize_x(const float *x, int ldx, int cols, int batch, int np, uint8_t *dig, float2 *meta,
     hipStream_t stream);
 
-// Batches above 8 with quantized weights: Q4_K / Q8_0 / Q4_0 on fp16 MFMA
-// (prefill_f16.hip), Q6_K on int8 MFMA (prefill.hip). The launch needs
+// Batches above 8 with quantized weights, on fp16 MFMA (prefill.hip chooses
+// between prefill_tile.hip and prefill_f16.hip). The launch needs
 // prefill_workspace bytes of 16-byte-aligned device scratch; prefill_kernel
 // names the GEMM kernel.
 size_t prefill_workspace(unsigned type, int cols, int batch);
@@ -103,7 +103,14 @@ hipError_t launch_prefill(unsigned type, const uint8_t *w, const float *x, float
     void *workspace, hipStream_t stream);
 const char *prefill_kernel(unsigned type);
 
-bool prefill_f16_supported(unsigned type);
+// Whole 256-column groups (prefill_tile.hip): every Q8_0, Q4_0 and Q6_K batch
+// of them, Q4_K batches that fill the chip. np: the tokens the workspace holds
+// pieces of (batch rounded up to a multiple of 32).
+bool prefill_tile_supported(unsigned type, int rows, int cols, int batch);
+hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
+    void *workspace, int np, hipStream_t s);
+// The other Q4_K batches, and Q8_0 / Q4_0 rows with a short last group
+// (prefill_f16.hip).
 size_t prefill_f16_workspace(int cols, int batch);
 hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
     int batch, void *workspace, hipStream_t stream);

@@ -1,5 +1,8 @@
 // Prefill GEMM Y[m][row] = sum_k W[row][k] * X[m][k] for batches above 8 on
-// gfx950 fp16 MFMA (v_mfma_f32_32x32x16_f16), Q4_K / Q8_0 / Q4_0 weights.
+// gfx950 fp16 MFMA (v_mfma_f32_32x32x16_f16): Q4_K batches too small to fill
+// the chip with the 256 x 64 workgroups of prefill_tile.hip, and Q8_0 / Q4_0
+// rows whose last 256-column group is short. Also splits the activations for
+// both files.
 //
 // Numbers. The weights enter the MFMA as exact fp16 integers: Q4_K sc * q
 // (<= 63 * 15 = 945), Q8_0 q, Q4_0 q - 8. Each token's activations are scaled
@@ -37,6 +40,7 @@
 
 #include "blockdot.h"
 #include "kernels.h"
+#include "pieces.h"
 
 namespace fy {
 namespace {
@@ -53,28 +57,7 @@ constexpr int kTileBytes = 2 * kPieceBytes + kSumBytes;   // one token tile of o
 // One LDS buffer holds a group for the workgroup's TW token tiles.
 template <int TW> constexpr int kBufBytes = TW * kTileBytes;
 
-// ---- activation pieces ---------------------------------------------------
-// Workspace for np tokens (np a multiple of 32): hi[np][cols], lo[np][cols]
-// (fp16, permuted as above), bsum[np][cols / 256][2][8] (the sum of x s over
-// 32-column block j of each 256-column group, times 2^-5, as two fp16
-// pieces: [0][j] hi, [1][j] lo; |sum| < 2^19, so the scaled sum is below the
-// fp16 range limit; written when cols % 256 == 0) and inv[np] (1 / s, or
-// NaN).
-struct Pieces {
-    _Float16 *hi, *lo, *bsum;
-    float *inv;
-};
-
-__host__ __device__ inline Pieces pieces_of(void *ws, int cols, int np)
-{
-    Pieces p;
-    p.hi = (_Float16 *)ws;
-    p.lo = p.hi + (size_t)np * cols;
-    p.bsum = p.lo + (size_t)np * cols;
-    p.inv = (float *)(p.bsum + (size_t)np * (cols / 16));
-    return p;
-}
-
+// ---- activation pieces (pieces.h) -----------------------------------------
 __device__ __forceinline__ float block_max(float v, float *red)
 {
 #pragma unroll
@@ -86,7 +69,9 @@ __device__ __forceinline__ float block_max(float v, float *red)
     return v;
 }
 
-// One workgroup per token; cols % 32 == 0.
+// One workgroup per token; cols % 32 == 0. TILED: the layout of tiled_block
+// and tiled_sums (cols % 256 == 0).
+template <bool TILED>
 __global__ __launch_bounds__(256) void split_x(const float *__restrict__ x, int cols, Pieces out)
 {
     __shared__ float red[4];
@@ -123,8 +108,10 @@ __global__ __launch_bounds__(256) void split_x(const float *__restrict__ x, int 
             hi[i] = (_Float16)v[i];
             lo[i] = (_Float16)(v[i] - (float)hi[i]);
         }
-        *(h8 *)(out.hi + (size_t)t * cols + 8 * c) = hi;
-        *(h8 *)(out.lo + (size_t)t * cols + 8 * c) = lo;
+        const size_t at = TILED ? ((size_t)(t / 32) * (cols / 128) + c / 16) * 4096 + 128 * (t % 32) + 8 * (c % 16)
+                                : (size_t)t * cols + 8 * c;
+        *(h8 *)(out.hi + at) = hi;
+        *(h8 *)(out.lo + at) = lo;
         // Four consecutive chunks form a 32-column block (256 is a multiple of 4).
         s += __shfl_xor(s, 1, 64);
         s += __shfl_xor(s, 2, 64);
@@ -132,9 +119,10 @@ __global__ __launch_bounds__(256) void split_x(const float *__restrict__ x, int 
             const int b = c / 4, j = b & 7;
             const float sv = s * 0.03125f;
             const _Float16 shi = (_Float16)sv;
-            _Float16 *dst = out.bsum + (size_t)t * (cols / 16) + 2 * (b & ~7) + j;
+            _Float16 *dst = TILED ? tiled_sums(out.bsum, cols, t, b >> 3) + 8 * (t % 32) + j
+                                  : out.bsum + (size_t)t * (cols / 16) + 2 * (b & ~7) + j;
             dst[0] = shi;
-            dst[8] = (_Float16)(sv - (float)shi);
+            dst[TILED ? 256 : 8] = (_Float16)(sv - (float)shi);
         }
     }
 }
@@ -252,16 +240,16 @@ __device__ __forceinline__ h8 b_operand(const WStage<T> &w, int j, int kappa, in
 }
 
 // Weight loads of one stage (the layout of formats.h, as load_weights in
-// blockdot.h reads it), as raw buffer loads over the tile. FULLK (every
-// group of the row a full 256-column group): always exactly kWeightLoads of
-// them; the wait before each barrier leaves that many in flight and counts
-// on them being the last vector memory instructions, so that it covers every
-// copy issued before them. Rows with a short last Q8_0/Q4_0 group issue
-// another count for that group and wait for all loads before each barrier.
-template <unsigned T, bool FULLK>
-constexpr int kWeightLoads = !FULLK ? 0 : T == Q8_0 ? 9 : 5;
+// blockdot.h reads it), as raw buffer loads over the tile. Q4_K (every group
+// of the row a full 256-column group): always exactly kWeightLoads of them;
+// the wait before each barrier leaves that many in flight and counts on them
+// being the last vector memory instructions, so that it covers every copy
+// issued before them. Rows with a short last Q8_0/Q4_0 group issue another
+// count for that group and wait for all loads before each barrier.
+template <unsigned T>
+constexpr int kWeightLoads = T == Q4_K ? 5 : 0;
 
-template <unsigned T, bool FULLK>
+template <unsigned T>
 __device__ __forceinline__ void load_stage(WStage<T> &w, __amdgpu_buffer_rsrc_t rs, const Lane &L, int g)
 {
     auto ld = [&](int off) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0)); };
@@ -284,19 +272,15 @@ __device__ __forceinline__ void load_stage(WStage<T> &w, __amdgpu_buffer_rsrc_t 
 #pragma unroll
             for (int k = 0; k < 8; ++k) w.d[k] = k < 4 ? d[k] : 0u;
         };
-        if constexpr (FULLK) {
+        const int nb = group_blocks(L, g);
+        if (nb == 8) {
             full();
         } else {
-            const int nb = group_blocks(L, g);
-            if (nb == 8) {
-                full();
-            } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int jj = j < nb ? j : nb - 1;
-                    w.q[j] = ld(b + quant * R * jj + (T == Q8_0 ? 16 * R * h : 0) + 16 * r);
-                    w.d[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, b + quant * R * nb + 2 * R * jj + 2 * r, 0, 0);
-                }
+            for (int j = 0; j < 8; ++j) {
+                const int jj = j < nb ? j : nb - 1;
+                w.q[j] = ld(b + quant * R * jj + (T == Q8_0 ? 16 * R * h : 0) + 16 * r);
+                w.d[j] = __builtin_amdgcn_raw_buffer_load_b16(rs, b + quant * R * nb + 2 * R * jj + 2 * r, 0, 0);
             }
         }
     }
@@ -311,7 +295,7 @@ __device__ __forceinline__ void load_stage(WStage<T> &w, __amdgpu_buffer_rsrc_t 
 // with another count of loads in flight. The two buffers come in as restrict
 // pointers, which lets the compiler see that this step's LDS reads do not
 // depend on the copies it issues.
-template <unsigned T, int RT, int TW, bool FULLK>
+template <unsigned T, int RT, int TW>
 __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], lds_u8 *__restrict__ buf,
     lds_u8 *__restrict__ nbuf, const Pieces &p, const Lane &L, __amdgpu_buffer_rsrc_t rs, int a_off, int cols, int m0,
     int g, int groups)
@@ -319,7 +303,7 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
     constexpr bool sums = T == Q4_K;
     // s_waitcnt immediate: vmcnt = kLoads (bits 3:0 and 15:14), expcnt and
     // lgkmcnt at their maxima (no wait).
-    constexpr int kLoads = kWeightLoads<T, FULLK>;
+    constexpr int kLoads = kWeightLoads<T>;
     constexpr int kWaitCopies = (kLoads & 15) | ((kLoads >> 4) << 14) | (7 << 4) | (15 << 8);
     static_assert(kLoads < 64, "vmcnt field");
     const int lane = threadIdx.x & 63;
@@ -433,10 +417,10 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
                     for (int r = 0; r < 16; ++r) acc[tt][r] += dj * C[tt][r];
             }
         };
-        if (FULLK || group_blocks(L, g) == 8) blocks(std::true_type{});
+        if (group_blocks(L, g) == 8) blocks(std::true_type{});
         else blocks(std::false_type{});
     }
-    load_stage<T, FULLK>(cur, rs, L, g + 2 < groups ? g + 2 : groups - 1);
+    load_stage<T>(cur, rs, L, g + 2 < groups ? g + 2 : groups - 1);
     // This wavefront's copies are complete; then every wavefront's are,
     // past the barrier. (The fence keeps the loads above before the wait.)
     asm volatile("" ::: "memory");
@@ -451,7 +435,7 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
 // of LDS, one workgroup per CU, 8 wavefronts of up to 256 VGPRs.
 // The weights are deliberately not a restrict pointer: the compiler may
 // then not move their loads across the memory fences of group_step.
-template <unsigned T, int RT, int TW, bool FULLK>
+template <unsigned T, int RT, int TW>
 __global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1 ? RT / 2 : RT / 4, TW == 1 ? RT / 2 : RT / 4))) void prefill_f16(
     const uint8_t *w, Pieces p, float *__restrict__ y, int rows, int cols, int batch, int token_blocks)
 {
@@ -488,8 +472,8 @@ __global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1
     // completed by an earlier step's wait).
     copy_group<RT, TW>(B0, p, cols, m0, 0, sums);
     asm volatile("" ::: "memory");
-    load_stage<T, FULLK>(st[0], rs, L, 0);
-    load_stage<T, FULLK>(st[1], rs, L, groups > 1 ? 1 : 0);
+    load_stage<T>(st[0], rs, L, 0);
+    load_stage<T>(st[1], rs, L, groups > 1 ? 1 : 0);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0);
     barrier();
@@ -507,27 +491,42 @@ __global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1
     // before each first step.
     int g = 0;
     for (; g + 1 < groups; g += 2) {
-        group_step<T, RT, TW, FULLK>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
-        group_step<T, RT, TW, FULLK>(st[1], acc, B1, B0, p, L, rs, a_off, cols, m0, g + 1, groups);
+        group_step<T, RT, TW>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
+        group_step<T, RT, TW>(st[1], acc, B1, B0, p, L, rs, a_off, cols, m0, g + 1, groups);
     }
-    if (g < groups) group_step<T, RT, TW, FULLK>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
+    if (g < groups) group_step<T, RT, TW>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
 
     if (tile_raw >= tiles || (lane & 31) >= R) return;
     const int row = kTileRows * tile + (lane & 31);
     // D register r of lane l is token 8 (r / 4) + 4 (l / 32) + r % 4 of its
-    // token tile.
+    // token tile. Every 1 / s is requested before the first store (loaded
+    // store by store they cost a memory round trip each).
+    float4 inv[TW][4];
+#pragma unroll
+    for (int tt = 0; tt < TW; ++tt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) inv[tt][q] = *(const float4 *)(p.inv + m0 + 32 * tt + 8 * q + 4 * L.h);
 #pragma unroll
     for (int tt = 0; tt < TW; ++tt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int t = 32 * tt + 8 * (r >> 2) + 4 * L.h + (r & 3);
-            if (t < n) y[(size_t)(m0 + t) * rows + row] = acc[tt][r] * p.inv[m0 + t];
+            const float4 v = inv[tt][r >> 2];
+            const float scale = (r & 3) == 0 ? v.x : (r & 3) == 1 ? v.y : (r & 3) == 2 ? v.z : v.w;
+            if (t < n) y[(size_t)(m0 + t) * rows + row] = acc[tt][r] * scale;
         }
 }
 
 }  // namespace
 
-bool prefill_f16_supported(unsigned type) { return type == Q4_K || type == Q8_0 || type == Q4_0; }
+hipError_t launch_split_x(const float *x, int batch, int cols, const Pieces &p, bool tiled, hipStream_t s)
+{
+    if (tiled)
+        hipLaunchKernelGGL(split_x<true>, dim3((unsigned)batch), dim3(256), 0, s, x, cols, p);
+    else
+        hipLaunchKernelGGL(split_x<false>, dim3((unsigned)batch), dim3(256), 0, s, x, cols, p);
+    return hipGetLastError();
+}
 
 // The pieces of the batch rounded up to 64 tokens (whole token blocks of
 // either kernel shape).
@@ -542,13 +541,12 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
 {
     const int np = (batch + 2 * kTokens - 1) / (2 * kTokens) * (2 * kTokens);
     const Pieces p = pieces_of(workspace, cols, np);
-    hipLaunchKernelGGL(split_x, dim3((unsigned)batch), dim3(256), 0, s, x, cols, p);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_split_x(x, batch, cols, p, false, s);
     if (e != hipSuccess) return e;
     const int tiles = (rows + kTileRows - 1) / kTileRows;
-    const bool fullk = cols % kGroupCols == 0;
     // Two token tiles per wavefront (each weight operand serves four MFMAs)
-    // where one workgroup per CU of 256 rows x 64 tokens fills the chip.
+    // where one workgroup per CU of 256 rows x 64 tokens fills the chip (Q4_K
+    // batches that do are prefill_tile.hip's).
     const int tb2 = (batch + 2 * kTokens - 1) / (2 * kTokens);
     const int tb = (batch + kTokens - 1) / kTokens;
     const bool pair = (tiles + 7) / 8 * tb2 >= 256;
@@ -557,25 +555,21 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
     const bool wide = type == Q4_K && (tiles + 7) / 8 * tb >= 256;
     const dim3 grid2((unsigned)((tiles + 7) / 8 * tb2));
     const dim3 grid((unsigned)((tiles + (wide ? 7 : 3)) / (wide ? 8 : 4) * tb));
-#define FY_PREFILL(TT, RTT, TWW, FK, G, TB) \
-    hipLaunchKernelGGL((prefill_f16<TT, RTT, TWW, FK>), G, dim3(64 * RTT), 0, s, w, p, y, rows, cols, batch, TB)
+#define FY_PREFILL(TT, RTT, TWW, G, TB) \
+    hipLaunchKernelGGL((prefill_f16<TT, RTT, TWW>), G, dim3(64 * RTT), 0, s, w, p, y, rows, cols, batch, TB)
     switch (type) {
     case Q4_K:
-        if (pair) FY_PREFILL(Q4_K, 8, 2, true, grid2, tb2);
-        else if (wide) FY_PREFILL(Q4_K, 8, 1, true, grid, tb);
-        else FY_PREFILL(Q4_K, 4, 1, true, grid, tb);
+        if (pair) FY_PREFILL(Q4_K, 8, 2, grid2, tb2);
+        else if (wide) FY_PREFILL(Q4_K, 8, 1, grid, tb);
+        else FY_PREFILL(Q4_K, 4, 1, grid, tb);
         break;
     case Q8_0:
-        if (pair && fullk) FY_PREFILL(Q8_0, 8, 2, true, grid2, tb2);
-        else if (pair) FY_PREFILL(Q8_0, 8, 2, false, grid2, tb2);
-        else if (fullk) FY_PREFILL(Q8_0, 4, 1, true, grid, tb);
-        else FY_PREFILL(Q8_0, 4, 1, false, grid, tb);
+        if (pair) FY_PREFILL(Q8_0, 8, 2, grid2, tb2);
+        else FY_PREFILL(Q8_0, 4, 1, grid, tb);
         break;
     case Q4_0:
-        if (pair && fullk) FY_PREFILL(Q4_0, 8, 2, true, grid2, tb2);
-        else if (pair) FY_PREFILL(Q4_0, 8, 2, false, grid2, tb2);
-        else if (fullk) FY_PREFILL(Q4_0, 4, 1, true, grid, tb);
-        else FY_PREFILL(Q4_0, 4, 1, false, grid, tb);
+        if (pair) FY_PREFILL(Q4_0, 8, 2, grid2, tb2);
+        else FY_PREFILL(Q4_0, 4, 1, grid, tb);
         break;
     default: return hipErrorInvalidValue;
     }

@@ -60,6 +60,33 @@ def test_batch_and_row_tails(compute, oracle, type_id, batch):
         check_rows(oracle, w, type_id, x[token], rows, cols, y[token])
 
 
+# One shape per workgroup form of the whole-group GEMM, with ragged rows and
+# tokens and group counts around the four-step rotation of the narrow forms
+# (rows, cols, batch): 64 x 32, 128 x 32, 128 x 64, 256 x 64.
+TILE_FORMS = [(200, 256, 33), (75, 512, 40), (300, 768, 65), (33, 1280, 97), (2081, 1024, 513), (4097, 512, 161),
+              (4000, 1280, 129), (8161, 256, 200), (8161, 768, 200), (16100, 512, 300), (33001, 256, 170)]
+
+
+@pytest.mark.parametrize("type_id", QUANT, ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols,batch", TILE_FORMS, ids=[f"{r}x{c}-n{b}" for r, c, b in TILE_FORMS])
+def test_prefill_workgroup_forms(compute, oracle, type_id, rows, cols, batch):
+    """Every token's whole output against float64 sums of the decoded weights
+    (the contract bound per row: 1e-6 (1 + sum |w x|), the bound the other
+    prefill tests check) and relative L2 1e-6: two fp16 pieces hold x to
+    2^-22, the sums are fp32."""
+    seed = type_id * 31 + rows + cols + batch
+    w = synth.weights(type_id, rows, cols, seed)
+    x = synth.activations(batch, cols, seed)
+    out = np.full(batch * rows + 2, 12345, dtype=np.float32)
+    print(f"prefill form {TYPE_NAMES[type_id]} {rows}x{cols} batch {batch}", flush=True)
+    compute.matmul_typed(w, rows, cols, type_id, x, batch, out=out[1:-1])
+    assert out[0] == 12345 and out[-1] == 12345
+    y = out[1:-1].reshape(batch, rows)
+    s, m = oracle.contract_sums(w, type_id, x, rows, cols)
+    assert np.all(np.abs(y - s) <= 1e-6 * (1 + m))
+    assert rel_l2(y, s) <= 1e-6
+
+
 @pytest.fixture(scope="module")
 def hip():
     from fyodor_amd.hip import Kernels, Runtime
