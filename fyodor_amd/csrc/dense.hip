@@ -82,27 +82,46 @@ hipError_t launch_type(const uint8_t *w, const float *x, float *y, int rows, int
     }
 }
 
-// ---- batches above 8: a GEMM on the fp32 matrix cores ----------------------
+// ---- batches above 8: a GEMM on the bf16 matrix cores ----------------------
 //
-// Y [batch][rows] = X [batch][cols] W^T on v_mfma_f32_32x32x2_f32: every
-// product of an fp32 activation and a weight (F16 and BF16 widen to fp32
-// exactly) is formed and accumulated in fp32, as the reference's CUDA GEMM
-// does (CUDA/gemm.cu:53-96), but on the matrix cores. A workgroup of four
-// wavefronts owns 64 tokens x 128 rows; wavefront w computes the 64 tokens
-// of rows 32 w .. 32 w + 31 as two 32 x 32 tiles, each in two accumulator
-// chains (even and odd column chunks) added at the end. K advances 32
-// columns per step: the workgroup stages the tokens' 64 x 32 and the rows'
-// 128 x 32 fp32 tiles in LDS (rows padded to 36 floats: conflict-free
-// 16-byte reads), and prefetches the next step's tiles into registers while
-// the matrix cores work on the current one. MFMA step s of a 32-column chunk
-// takes column 16 h + s in lane half h, for both operands alike. Tokens past
-// the batch and rows past the matrix read zeros (buffer range checks); the
-// columns of a short last chunk (or of rows not 16-byte aligned) are loaded
-// one by one with their bounds.
-constexpr int kGemmTokens = 64, kGemmRows = 128, kGemmK = 32, kGemmPitch = 36;
+// Y [batch][rows] = X [batch][cols] W^T with fp32 products and accumulation,
+// as the reference's CUDA GEMM (CUDA/gemm.cu:53-96), on
+// v_mfma_f32_32x32x16_bf16: an fp32 value is exactly the sum of three bf16
+// ones (each the rounded rest of the ones before), an F16 weight of two, a BF16
+// weight is one. Products of bf16 pairs are exact in the MFMA, so
+//   BF16  w x = w x1 + w x2 + w x3                               (3 MFMAs)
+//   F16   w x = w1 x1 + (w1 x2 + w2 x1) + (w1 x3 + w2 x2) + e    (5)
+//   F32   w x = the same + w3 x1 + e                             (6)
+// with |e| below 2^-24 |w x|: the error of one fp32 product. The leading
+// products have an accumulator of their own, so the others round at 2^-8 of
+// its scale. 32 x 32 x 16 takes 96, 160 or 192 cycles where the fp32 matrix
+// cores take 512 (153 TFLOP/s measured for a library fp32 product).
+//
+// The matrix cores read bf16 subnormals as zeros, so that a product loses up
+// to about 2^-125 (|w| + |x|), and a non-finite value, or one that rounds to
+// infinity, leaves NaN or infinity in its outputs. Outputs small enough for the
+// first to show (against the largest operand that the workgroup met) or not
+// finite are computed again as plain fp32 dots.
+//
+// Work split. A workgroup of eight wavefronts owns 64 tokens x 128 rows;
+// wavefront (wr, ks) computes the 64 tokens of rows 32 wr .. 32 wr + 31 over
+// the ks-th half of the columns (two wavefronts per SIMD, and sums half as
+// long), 64 columns per step. The weights go from memory to their operand
+// registers and are split there; the tokens' pieces are made once per
+// workgroup half and read from LDS by its four wavefronts, double-buffered
+// with one barrier per step; 16-byte chunk c of token t at place c ^ (t / 2 % 8).
+// Tokens past the batch and rows past the matrix read zeros (buffer range
+// checks).
+//
+// 4096 x 4096, us before (fp32 matrix cores) and now: see launch_gemm.
+constexpr int kGemmTokens = 64, kGemmRows = 128, kGemmK = 64;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 template <unsigned T> constexpr int kElem = T == F32 ? 4 : 2;
+template <unsigned T> constexpr int kPieces = T == F32 ? 3 : T == F16 ? 2 : 1;   // of a weight
+constexpr int kPlaneBytes = kGemmTokens * kGemmK * 2;   // one piece of a step's tokens
 
 template <unsigned T>
 __device__ __forceinline__ float widen(uint32_t bits)
@@ -111,153 +130,321 @@ __device__ __forceinline__ float widen(uint32_t bits)
     else return bf16_to_f32(bits & 0xFFFFu);
 }
 
-// Thread t's share of a step: W row t/2, columns 16 (t%2) .. +15; X token
-// t/4, columns 8 (t%4) .. +7 (as fp32).
-struct GemmStage {
-    float w[16];
-    float x[8];
-};
-
-template <unsigned T>
-__device__ __forceinline__ void gemm_load(GemmStage &st, __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb,
-    int rows, int cols, int batch, int r0, int t0, int kc, bool fast)
+// N bf16 pieces of each of 2 P values, packed in pairs.
+template <int N, int P>
+__device__ __forceinline__ void split(const float (&v)[2 * P], uint32_t (&out)[N][P])
 {
-    const int t = threadIdx.x;
-    const int row = r0 + (t >> 1), wcol = kc + 16 * (t & 1);
-    const int tok = t0 + (t >> 2), xcol = kc + 8 * (t & 3);
-    if (fast) {
-        // Whole chunk, 16-byte aligned rows.
-        const int wo = (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)wcol) * kElem<T>);
-        if constexpr (T == F32) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(wb, wo + 16 * q, 0, 0));
-                st.w[4 * q] = v.x; st.w[4 * q + 1] = v.y; st.w[4 * q + 2] = v.z; st.w[4 * q + 3] = v.w;
+    for (int i = 0; i < P; ++i) {
+        float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+            out[p][i] = __builtin_bit_cast(uint32_t, (bf16x2){(__bf16)a, (__bf16)b});
+            if (p + 1 < N) {
+                a = a - __builtin_bit_cast(float, out[p][i] << 16);
+                b = b - __builtin_bit_cast(float, out[p][i] & 0xFFFF0000u);
             }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wb, wo + 16 * q, 0, 0));
-                const uint32_t u[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    st.w[8 * q + 2 * e] = widen<T>(u[e]);
-                    st.w[8 * q + 2 * e + 1] = widen<T>(u[e] >> 16);
-                }
-            }
-        }
-        const int xo = (int)(((uint32_t)tok * (uint32_t)cols + (uint32_t)xcol) * 4u);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xb, xo + 16 * q, 0, 0));
-            st.x[4 * q] = v.x; st.x[4 * q + 1] = v.y; st.x[4 * q + 2] = v.z; st.x[4 * q + 3] = v.w;
-        }
-    } else {
-        // Element by element, zero past the row's last column.
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int c = wcol + e;
-            const int off = (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)(c < cols ? c : 0)) * kElem<T>);
-            float v;
-            if constexpr (T == F32) v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wb, off, 0, 0));
-            else v = widen<T>(__builtin_amdgcn_raw_buffer_load_b16(wb, off, 0, 0));
-            st.w[e] = c < cols ? v : 0.f;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int c = xcol + e;
-            const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                xb, (int)(((uint32_t)tok * (uint32_t)cols + (uint32_t)(c < cols ? c : 0)) * 4u), 0, 0));
-            st.x[e] = c < cols ? v : 0.f;
         }
     }
-    (void)rows;
-    (void)batch;
 }
 
-__device__ __forceinline__ void gemm_store(const GemmStage &st, float *__restrict__ sw, float *__restrict__ sx)
+// This lane's weights of a step as loaded: slice s (of four) holds columns
+// 16 s + 8 h .. + 7 of its row (the two lanes of a row read 32 or 64
+// consecutive bytes per slice). ALIGNED: rows 16-byte aligned, else element by
+// element. Columns past the row's end hold whatever follows (the buffer range
+// bounds it): their activations are zeros, and where a product of zero is no
+// number the output is computed again.
+template <unsigned T>
+struct GemmWeights {
+    u32x4 w[T == F32 ? 8 : 4];
+};
+
+// Slice s of the step at column kc.
+template <unsigned T, bool ALIGNED>
+__device__ __forceinline__ void load_slice(GemmWeights<T> &st, __amdgpu_buffer_rsrc_t wb, int cols, int row, int kc, int s)
 {
-    const int t = threadIdx.x;
-    float *dw = sw + (t >> 1) * kGemmPitch + 16 * (t & 1);
+    constexpr int kPer = T == F32 ? 2 : 1;   // 16-byte words per slice
+    const int h = (int)((threadIdx.x >> 5) & 1);
+    const int at = (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)(kc + 16 * s + 8 * h)) * kElem<T>);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        *(float4 *)(dw + 4 * q) = make_float4(st.w[4 * q], st.w[4 * q + 1], st.w[4 * q + 2], st.w[4 * q + 3]);
-    float *dx = sx + (t >> 2) * kGemmPitch + 8 * (t & 3);
+    for (int q = 0; q < kPer; ++q) {
+        if constexpr (ALIGNED) {
+            st.w[kPer * s + q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, at + 16 * q, 0, 0));
+        } else {
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-        *(float4 *)(dx + 4 * q) = make_float4(st.x[4 * q], st.x[4 * q + 1], st.x[4 * q + 2], st.x[4 * q + 3]);
+            for (int e = 0; e < 4; ++e) {
+                const int off = at + 16 * q + 4 * e;
+                st.w[kPer * s + q][e] = T == F32 ? __builtin_amdgcn_raw_buffer_load_b32(wb, off, 0, 0)
+                                                 : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wb, off, 0, 0) |
+                                                       (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wb, off + 2, 0, 0) << 16;
+            }
+        }
+    }
 }
 
-// Workgroup (row tile, token tile, split z) covers the column chunks
+// This thread's sixteen activations of a step: columns 4 (l % 16) .. + 3 of
+// tokens 16 (wave % 4) + 4 q + l / 16, q = 0..3 (a load covers 256 consecutive
+// bytes of four tokens).
+struct Tokens {
+    int first, col;   // the first token (of the workgroup's 64), the column within a step
+};
+
+__device__ __forceinline__ Tokens tokens_of()
+{
+    const int t = threadIdx.x & 255;
+    return {16 * (t >> 6) + ((t & 63) >> 4), 4 * (t & 15)};
+}
+
+template <bool ALIGNED>
+__device__ __forceinline__ void load_tokens(float (&x)[16], __amdgpu_buffer_rsrc_t xb, int cols, int t0, int kc)
+{
+    const Tokens t = tokens_of();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int at = (int)(((uint32_t)(t0 + t.first + 4 * q) * (uint32_t)cols + (uint32_t)(kc + t.col)) * 4u);
+        if constexpr (ALIGNED) {
+            const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xb, at, 0, 0));
+            x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                x[4 * q + e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xb, at + 4 * e, 0, 0));
+        }
+    }
+}
+
+// Zeros for the columns from kend on (a uniform test: whole steps skip it).
+__device__ __forceinline__ void cut_tokens(float (&x)[16], int kc, int kend)
+{
+    if (kc + kGemmK <= kend) return;
+    const int col = kc + tokens_of().col;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = col + i % 4 < kend ? x[i] : 0.f;
+}
+
+__device__ __forceinline__ float larger(float m, float a, float b)
+{
+    return __builtin_fmaxf(m, __builtin_fmaxf(__builtin_fabsf(a), __builtin_fabsf(b)));
+}
+
+// The pieces of two of its tokens (half 0 or 1) into LDS: plane p at
+// p kPlaneBytes, token t's 128 bytes at 128 t.
+__device__ __forceinline__ void store_tokens(const float (&x)[16], int half, uint8_t *lds, float &big)
+{
+    const Tokens t = tokens_of();
+#pragma unroll
+    for (int q = 2 * half; q < 2 * half + 2; ++q) {
+        const float v[4] = {x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+        big = larger(larger(big, v[0], v[1]), v[2], v[3]);
+        uint32_t p[3][2];
+        split<3, 2>(v, p);
+        const int token = t.first + 4 * q, at = 128 * token + 16 * ((t.col >> 3) ^ ((token >> 1) & 7)) + 2 * (t.col & 4);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *(uint2 *)(lds + k * kPlaneBytes + at) = make_uint2(p[k][0], p[k][1]);
+    }
+}
+
+// Slice s in pieces; big becomes the largest magnitude met (a BF16 pair's
+// second value is taken with the first one's bits below it; F16 stays below
+// the 2^16 that big starts from).
+template <unsigned T>
+__device__ __forceinline__ void weight_pieces(const GemmWeights<T> &st, int s, bf16x8 (&out)[kPieces<T>], float &big)
+{
+    if constexpr (T == BF16) {
+        out[0] = __builtin_bit_cast(bf16x8, st.w[s]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t word = st.w[s][i];
+            big = larger(big, __builtin_bit_cast(float, word << 16), __builtin_bit_cast(float, word));
+        }
+    } else {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            // A copy first: a bit cast of the vector's element reads element 0.
+            const uint32_t word = T == F32 ? st.w[(2 * s + i / 4) % (T == F32 ? 8 : 4)][i % 4] : st.w[s][i / 2];
+            if constexpr (T == F32) v[i] = __builtin_bit_cast(float, word);
+            else v[i] = widen<T>(word >> (16 * (i & 1)));
+        }
+        if constexpr (T == F32) {
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) big = larger(big, v[i], v[i + 1]);
+        }
+        uint32_t p[kPieces<T>][4];
+        split<kPieces<T>, 4>(v, p);
+#pragma unroll
+        for (int k = 0; k < kPieces<T>; ++k)
+            out[k] = __builtin_bit_cast(bf16x8, (u32x4){p[k][0], p[k][1], p[k][2], p[k][3]});
+    }
+}
+
+// One output as a plain fp32 dot over columns [k0, k1), by the wavefront.
+template <unsigned T>
+__device__ float plain_dot(const uint8_t *w, const float *x, int cols, int row, int token, int k0, int k1)
+{
+    const float *xr = x + (size_t)token * cols;
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = k0 + (int)(threadIdx.x & 63); k < k1; k += 64) {
+        const size_t at = (size_t)row * cols + k;
+        float wv;
+        if constexpr (T == F32) wv = ((const float *)w)[at];
+        else wv = widen<T>(((const uint16_t *)w)[at]);
+        s += wv * xr[k];
+    }
+    return wave_sum(s);
+}
+
+// Workgroup (row tile, token tile, split z) covers the 64-column steps
 // [z per, (z + 1) per) of the split count gridDim.z; with one split it
 // writes Y, else its partial sums to part[z][token][row] for dense_combine.
-template <unsigned T>
-__global__ __launch_bounds__(256) void dense_gemm(const uint8_t *__restrict__ w, const float *__restrict__ x,
-    float *__restrict__ y, int rows, int cols, int batch, int per, float *__restrict__ part)
+template <unsigned T, bool ALIGNED>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_gemm(
+    const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int rows, int cols, int batch,
+    int per, float *__restrict__ part)
 {
-    __shared__ __align__(16) float sw[kGemmRows * kGemmPitch];
-    __shared__ __align__(16) float sx[kGemmTokens * kGemmPitch];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
+    constexpr int kBuf = 3 * kPlaneBytes;
+    __shared__ __align__(16) uint8_t sx[2][2][kBuf];   // [half of the columns][buffer]
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave & 3, ks = wave >> 2;
     const int r0 = blockIdx.x * kGemmRows, t0 = blockIdx.y * kGemmTokens;
     const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(w), (short)0, (int)((size_t)rows * cols * kElem<T>), 0x00020000);
     const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float *>(x), (short)0, (int)((size_t)batch * cols * 4), 0x00020000);
-    const bool aligned = (cols * kElem<T>) % 16 == 0;
-    // Two chains per output, even and odd chunks, added at the end (the
-    // reference's CUDA GEMM keeps two as well): partial sums stay half as
-    // long, which keeps sums like 8192 equal products exact.
-    f32x16 acc[2][2] = {};
-    int chain = 0;
-    GemmStage st;
     const int k0 = blockIdx.z * per * kGemmK, k1 = k0 + per * kGemmK < cols ? k0 + per * kGemmK : cols;
-    if (k0 < k1) gemm_load<T>(st, wb, xb, rows, cols, batch, r0, t0, k0, aligned && k0 + kGemmK <= cols);
-    for (int kc = k0; kc < k1; kc += kGemmK) {
-        __syncthreads();   // the previous step's operand reads are done
-        gemm_store(st, sw, sx);
+    // Both halves walk as many steps (the barriers are the workgroup's); past
+    // its columns the second one's loads are zeros.
+    const int steps = k0 < k1 ? ((k1 - k0 + kGemmK - 1) / kGemmK + 1) / 2 : 0;
+    const int first = k0 + ks * steps * kGemmK, mid = k0 + steps * kGemmK, kend = ks || k1 < mid ? k1 : mid;
+    const int row = r0 + 32 * wr + (lane & 31);
+    // Leading products and the rest, per token tile.
+    f32x16 acc[2][2] = {};
+    // Step i takes each slice's weights out of their registers and requests
+    // step i + 2's into them; meanwhile the tokens of step i + 1, requested in
+    // step i - 1, are split into the other buffer, and those of step i + 2
+    // requested.
+    float big = T == F16 ? 0x1p16f : 0.f;   // the largest |w| and |x| met
+    GemmWeights<T> w0, w1;
+    float x0[16], x1[16];
+    auto at = [&](int i) { return first + i * kGemmK; };
+    auto step = [&](int i, int odd, GemmWeights<T> &cur, float (&xs)[16], float (&xn)[16]) {
+        // (Past the last step nobody computes on what is requested.)
+        load_tokens<ALIGNED>(xn, xb, cols, t0, at(i + 2));
+        __builtin_amdgcn_sched_barrier(0);
+        cut_tokens(xs, at(i + 1), kend);
+        const uint8_t *buf = sx[ks][odd];
+        bf16x8 a[2][2][3], b[2][kPieces<T>];
+        auto fetch = [&](int s, bf16x8 (&x8)[2][3], bf16x8 (&w8)[kPieces<T>]) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    x8[t][p] = *(const bf16x8 *)(buf + p * kPlaneBytes + 128 * (32 * t + (lane & 31)) +
+                                                 16 * ((2 * s + h) ^ ((lane >> 1) & 7)));
+            weight_pieces<T>(cur, s, w8, big);
+        };
+        // A slice's operands are made among the MFMAs of the one before, but
+        // for F32, whose second set would not fit the registers.
+        constexpr bool kAhead = T != F32;
+        if (kAhead) fetch(0, a[0], b[0]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (!kAhead) fetch(s, a[s & 1], b[s & 1]);
+            else if (s < 3) fetch(s + 1, a[(s + 1) & 1], b[(s + 1) & 1]);
+            if (s < 2) store_tokens(xs, s, sx[ks][1 - odd], big);
+            // The two token tiles in turn.
+            auto mul = [&](int which, int pa, int pb) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    acc[t][which] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][t][pa], b[s & 1][pb], acc[t][which],
+                                                                            0, 0, 0);
+            };
+            mul(1, 2, 0);
+            mul(0, 0, 0);
+            mul(1, 1, 0);
+            if constexpr (kPieces<T> > 1) {
+                mul(1, 1, 1);
+                mul(1, 0, 1);
+            }
+            if constexpr (kPieces<T> > 2) mul(1, 0, 2);
+            load_slice<T, ALIGNED>(cur, wb, cols, row, at(i + 2), s);
+            constexpr int kMfma = 2 * (kPieces<T> == 1 ? 3 : kPieces<T> == 2 ? 5 : 6);
+#pragma unroll
+            for (int q = 0; q < kMfma; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // VALU
+                if (q < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+            }
+            __builtin_amdgcn_sched_group_barrier(0x020, T == F32 ? 2 : 1, 0);   // the slice's load
+        }
         __syncthreads();
-        const int kn = kc + kGemmK;
-        if (kn < k1) gemm_load<T>(st, wb, xb, rows, cols, batch, r0, t0, kn, aligned && kn + kGemmK <= cols);
-        // This lane's operands: row 32 wave + l%32 and tokens l%32, 32 + l%32,
-        // columns 16 h .. 16 h + 15 of the chunk.
-        const float *pw = sw + (32 * wave + (lane & 31)) * kGemmPitch + 16 * h;
-        const float *px0 = sx + (lane & 31) * kGemmPitch + 16 * h;
-        const float *px1 = px0 + 32 * kGemmPitch;
-        float bw[16], a0[16], a1[16];
+    };
+    if (steps) {
+        load_tokens<ALIGNED>(x0, xb, cols, t0, at(0));
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 vw = *(const float4 *)(pw + 4 * q), v0 = *(const float4 *)(px0 + 4 * q),
-                         v1 = *(const float4 *)(px1 + 4 * q);
-            bw[4 * q] = vw.x; bw[4 * q + 1] = vw.y; bw[4 * q + 2] = vw.z; bw[4 * q + 3] = vw.w;
-            a0[4 * q] = v0.x; a0[4 * q + 1] = v0.y; a0[4 * q + 2] = v0.z; a0[4 * q + 3] = v0.w;
-            a1[4 * q] = v1.x; a1[4 * q + 1] = v1.y; a1[4 * q + 2] = v1.z; a1[4 * q + 3] = v1.w;
-        }
-        if (chain == 0) {
+        for (int s = 0; s < 4; ++s) load_slice<T, ALIGNED>(w0, wb, cols, row, at(0), s);
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], bw[s], acc[0][0], 0, 0, 0);
-                acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], bw[s], acc[1][0], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], bw[s], acc[0][1], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], bw[s], acc[1][1], 0, 0, 0);
-            }
-        }
-        chain ^= 1;
+        for (int s = 0; s < 4; ++s) load_slice<T, ALIGNED>(w1, wb, cols, row, at(1), s);
+        cut_tokens(x0, at(0), kend);
+        store_tokens(x0, 0, sx[ks][0], big);
+        store_tokens(x0, 1, sx[ks][0], big);
+        load_tokens<ALIGNED>(x0, xb, cols, t0, at(1));
     }
-    // D[token][row]: register i of lane l holds token 8 (i/4) + 4 h + i%4
-    // (of the accumulator's 32), row l%32.
-    const int row = r0 + 32 * wave + (lane & 31);
-    if (row >= rows) return;
+    __syncthreads();
+    // Two steps per pass: the registers of one take the loads of the next
+    // without copies (a copy would wait for them).
+    for (int i = 0; i + 1 < steps; i += 2) {
+        step(i, 0, w0, x0, x1);
+        step(i + 1, 1, w1, x1, x0);
+    }
+    if (steps & 1) step(steps - 1, 0, w0, x0, x1);
+    // The halves meet in LDS. D[token][row]: register i of lane l holds token
+    // 8 (i / 4) + 4 h + i % 4 of its token tile, row l % 32.
+    float *meet = (float *)&sx[0][0][0] + 2048 * wr + lane, *most = (float *)&sx[0][0][0] + 8192;
+    for (int o = 32; o; o >>= 1) big = __builtin_fmaxf(big, __shfl_xor(big, o, 64));
+    if (lane == 0) most[wave] = big;
+    if (ks == 1) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) meet[64 * (16 * t + i)] = acc[t][0][i] + acc[t][1][i];
+    }
+    __syncthreads();
+    if (ks == 1) return;
+    for (int i = 0; i < 8; ++i) big = __builtin_fmaxf(big, most[i]);
+    // cols 2^-125 2 big is lost at most; it may weigh 2^-25.
+    const float least = (float)cols * 0x1p-99f * big;
     float *out = gridDim.z == 1 ? y : part + (size_t)blockIdx.z * batch * rows;
+    auto token = [&](int i) { return t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3); };
+    uint32_t again = 0;
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int tok = t0 + 32 * a + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (tok < batch) out[(size_t)tok * rows + row] = acc[a][0][i] + acc[a][1][i];
+    for (int i = 0; i < 32; ++i) {
+        const float v = (acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15]) + meet[64 * i];
+        if (row < rows && token(i) < batch) {
+            const float m = __builtin_fabsf(v);
+            if (!(m >= least && m <= 3.402823466e38f)) again |= 1u << i;
+            out[(size_t)token(i) * rows + row] = v;
+        }
+    }
+    if (__ballot(again != 0) == 0) return;
+    for (int i = 0; i < 32; ++i)
+        for (int half = 0; half < 2; ++half) {
+            uint64_t need = __ballot(again >> i & 1) & 0xFFFFFFFFull << 32 * half;
+            if (need == 0) continue;
+            const int tok = __builtin_amdgcn_readlane(token(i), 32 * half);
+            // The zeros of a token of zeros stand.
+            bool any = false;
+#pragma unroll 16
+            for (int k = k0 + lane; k < k1; k += 64) any |= x[(size_t)tok * cols + k] != 0.f;
+            if (__ballot(any) == 0) need = __ballot((again >> i & 1) && out[(size_t)tok * rows + row] != 0.f) & need;
+            while (need) {
+                const int l = __ffsll((unsigned long long)need) - 1, at = __builtin_amdgcn_readlane(row, l);
+                need &= need - 1;
+                const float v = plain_dot<T>(w, x, cols, at, tok, k0, k1);
+                if (lane == l) out[(size_t)tok * rows + at] = v;
+            }
         }
 }
 
@@ -272,14 +459,27 @@ __global__ __launch_bounds__(256) void dense_combine(const float *__restrict__ p
     }
 }
 
+// us before (one fp32 MFMA chain, 64 x 64 tiles) and now, 4096 x 4096 by
+// tokens, alone on the stream:
+//          16          333          512          2048
+//   F16    38 -> 18    219 -> 70    235 -> 83    690 -> 335
+//   BF16   38 -> 18    243 -> 64    241 -> 67
+//   F32    34 -> 28    208 -> 112   213 -> 115
+// At 512 tokens that is 1030 (F16), 770 (BF16) and 900 (F32) TFLOP/s issued
+// of the 1406 a large bf16 product reaches here: what bounds it now. Rows of
+// a multiple of 16 bytes load 16 bytes per lane; the others element by
+// element (F32 300 x 1002, 300 tokens: 39 -> 16.5 us).
 template <unsigned T>
 hipError_t launch_gemm(const uint8_t *w, const float *x, float *y, int rows, int cols, int batch, int splits,
     float *part, hipStream_t s)
 {
-    const int chunks = (cols + kGemmK - 1) / kGemmK, per = (chunks + splits - 1) / splits;
+    const int steps = (cols + kGemmK - 1) / kGemmK, per = (steps + splits - 1) / splits;
     const dim3 grid((unsigned)((rows + kGemmRows - 1) / kGemmRows), (unsigned)((batch + kGemmTokens - 1) / kGemmTokens),
                     (unsigned)splits);
-    hipLaunchKernelGGL((dense_gemm<T>), grid, dim3(256), 0, s, w, x, y, rows, cols, batch, per, part);
+    if ((size_t)cols * kElem<T> % 16 == 0)
+        hipLaunchKernelGGL((dense_gemm<T, true>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
+    else
+        hipLaunchKernelGGL((dense_gemm<T, false>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
     if (splits > 1) {
         const size_t n = (size_t)batch * rows;
         const size_t blocks = (n + 255) / 256;
@@ -299,7 +499,7 @@ int dense_gemm_splits(int rows, int cols, int batch)
 {
     const long tiles = (long)((rows + kGemmRows - 1) / kGemmRows) * ((batch + kGemmTokens - 1) / kGemmTokens);
     int splits = 1;
-    while (splits < 8 && tiles * splits < 192 && (cols + kGemmK - 1) / kGemmK >= 16 * splits) splits *= 2;
+    while (splits < 8 && tiles * splits < 192 && (cols + 31) / 32 >= 16 * splits) splits *= 2;
     return splits;
 }
 
@@ -368,7 +568,6 @@ namespace {
 // read zeros (buffer range check); they stay live through an xor that is
 // stored only if it equals a constant.
 constexpr int kReadWaves = 4, kReadDepth = 32;
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(64 * kReadWaves) void read16(const uint8_t *__restrict__ src, size_t bytes, size_t share,
     unsigned *__restrict__ sink)
 {

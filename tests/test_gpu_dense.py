@@ -1,4 +1,4 @@
-"""Dense F32 / F16 / BF16 batches above 8 on the fp32-MFMA GEMM
+"""Dense F32 / F16 / BF16 batches above 8 on the matrix-core GEMM
 (nya_hip_matmul, kernel "dense_gemm"), through the kernel library's C ABI:
 
 - under the reference kernel contract (backend/tests/test_quant_kernels.c:13-25,
@@ -97,3 +97,68 @@ def test_dense_gemm_exact_integers(hip, t):
     for workspace in (True, False):
         y = run(hip, w, t, x, rows, cols, batch, workspace)
         assert np.array_equal(y.astype(np.float64), exact)
+
+
+def stored(t, v):
+    """fp32 values as stored type t (bytes) and the values it holds."""
+    if t == F32:
+        return v.view(np.uint8).reshape(-1).copy(), v
+    if t == F16:
+        h = v.astype(np.float16)
+        return h.view(np.uint8).reshape(-1).copy(), h.astype(np.float32)
+    h = (v.view(np.uint32) >> 16).astype(np.uint16)
+    return h.view(np.uint8).reshape(-1).copy(), (h.astype(np.uint32) << 16).view(np.float32)
+
+
+# Columns about the 64-column step, its halves between the two column groups
+# (an odd number of steps, one step, a step of one column) and unaligned rows;
+# tokens and rows about their tiles of 64 and 128.
+EDGES = [(127, 8, 9), (128, 63, 64), (1, 64, 65), (129, 65, 63), (130, 136, 9), (257, 192, 130), (5, 321, 66),
+         (128, 1096, 64), (128, 2184, 10)]
+
+
+@pytest.mark.parametrize("t", [F32, F16, BF16], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("wscale,xscale", [(0, 0), (-14, 90), (-112, 100), (100, -122)])
+def test_dense_gemm_pieces(hip, t, wscale, xscale):
+    """Values across the exponent range, weights and activations that take
+    every bit of their pieces. Products left out weigh below 2^-25 of their
+    own magnitude, and a sum of n / 16 partial results rounds at most that
+    often: (n / 16 + 16) 2^-24 of sum |w x|."""
+    if t == F16:
+        wscale = max(wscale, -14) if wscale < 0 else min(wscale, 12)
+    for rows, cols, batch in EDGES:
+        rng = np.random.default_rng(rows + cols + batch + t)
+        wv = np.ldexp(rng.uniform(-1, 1, (rows, cols)) * 2.0 ** rng.integers(-8, 1, (rows, cols)), wscale).astype(np.float32)
+        x = np.ldexp(rng.uniform(-1, 1, (batch, cols)) * 2.0 ** rng.integers(-8, 1, (batch, cols)), xscale).astype(np.float32)
+        w, wv = stored(t, wv)
+        exact = x.astype(np.float64) @ wv.astype(np.float64).T
+        bound = (cols / 16 + 16) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(wv).astype(np.float64).T)
+        for workspace in (True, False):
+            y = run(hip, w, t, x, rows, cols, batch, workspace)
+            bad = np.abs(y - exact) > bound
+            assert not bad.any(), (rows, cols, batch, workspace, int(bad.sum()))
+
+
+@pytest.mark.parametrize("t", [F32, F16, BF16], ids=lambda t: TYPE_NAMES[t])
+def test_dense_gemm_non_finite(hip, t):
+    """Infinities, NaN and the largest values give what a plain sum gives:
+    the same infinities and NaN in the same outputs, the others untouched."""
+    rows, cols, batch = 130, 200, 70
+    rng = np.random.default_rng(t + 1)
+    wv = rng.uniform(-1, 1, (rows, cols)).astype(np.float32)
+    x = rng.uniform(-1, 1, (batch, cols)).astype(np.float32)
+    wv[3, 199], wv[64, 0], wv[129, 100], wv[7, 50], wv[7, 51] = np.inf, -np.inf, np.nan, np.inf, np.inf
+    x[0, 64], x[9, 199], x[63, 5], x[69, 150] = np.inf, 0.0, -np.inf, np.nan
+    x[20], x[30], x[40:48] = 0.0, 1e-40, 0.0
+    x[20, 3], x[21, 4] = np.float32(3.4028235e38), np.float32(-3.4e38)
+    w, wv = stored(t, wv)
+    with np.errstate(invalid="ignore"):
+        exact = np.stack([[np.sum(x[b].astype(np.float64) * wv[r].astype(np.float64)) for r in range(rows)]
+                          for b in range(batch)])
+        m = np.stack([np.sum(np.abs(x[b].astype(np.float64) * wv.astype(np.float64)), axis=1) for b in range(batch)])
+    for workspace in (True, False):
+        y = run(hip, w, t, x, rows, cols, batch, workspace).astype(np.float64)
+        assert np.array_equal(np.isnan(y), np.isnan(exact))
+        finite = np.isfinite(exact)
+        assert np.array_equal(y[~finite & ~np.isnan(exact)], exact[~finite & ~np.isnan(exact)])
+        assert np.all(np.abs(y[finite] - exact[finite]) <= (cols / 16 + 16) * 2.0 ** -24 * m[finite])
