@@ -40,14 +40,12 @@ bool storage_bytes(unsigned type, size_t rows, size_t cols, size_t *bytes)
 
 // Batches above the small-N kernels' 8 columns go to the prefill GEMM (every
 // block format), except small batches of matrices the row-balanced small-N
-// kernel takes: those stay memory-bound, and launches of 8 tokens each beat
-// the GEMM's activation split and sparse grid up to a batch measured per
-// shape (MI355X, 50 calls over rotating weights, GEMM / 8-token launches):
-// Q4_K 14336 x 4096 at 16 tokens 32.0 / 22.3 us, at 24 32.6 / 33.0; Q4_K and
-// Q8_0 4096 x 4096 at 32 31.4 / 26.2 and 40.7 / 25.6, at 40 31.1 / 32.6;
-// Q6_K 4096 x 14336 (its int8 GEMM starts slow on wide rows) at 48
-// 203.9 / 152.7, at 64 203.9 / 201.9. The Q6_K output head (128256 x 4096)
-// keeps the GEMM from 9 tokens on (173 / 198 us).
+// kernel takes, which need no workspace and run on rows_tokens.hip or, 8
+// tokens per launch, on that kernel, up to a batch measured per shape (MI355X,
+// 50 calls over rotating weights, GEMM / 8-token launches): Q4_K 14336 x 4096
+// at 16 tokens 32.0 / 22.3 us, at 24 32.6 / 33.0; Q4_K and Q8_0 4096 x 4096 at
+// 32 31.4 / 26.2 and 40.7 / 25.6 (14.4 and 15.5 on rows_tokens.hip). The Q6_K
+// output head (128256 x 4096) keeps the GEMM from 9 tokens on (173 / 198 us).
 bool use_prefill(unsigned type, size_t rows, size_t cols, size_t batch)
 {
     if (batch <= 8 || !(type == Q4_K || type == Q6_K || type == Q8_0 || type == Q4_0)) return false;
@@ -82,33 +80,41 @@ int matmul_impl(uintptr_t w, unsigned type, size_t rows, size_t cols, uintptr_t 
     const uint8_t *wp = (const uint8_t *)w;
     const bool fits = workspace && !(workspace & 15u);
     // The GEMM needs its workspace; without one (or a short one) the batch is
-    // run 8 columns at a time instead.
+    // run up to 64 or 8 columns at a time instead.
     if (use_prefill(type, rows, cols, batch) && fits && workspace_bytes >= prefill_workspace(type, (int)cols, (int)batch))
         return status(launch_prefill(type, wp, (const float *)x, (float *)y, (int)rows, (int)cols, (int)batch,
                                      (void *)workspace, s));
     if (dense && dense_gemm_supported(type, (int)rows, (int)cols, (int)batch))
         return status(launch_dense_gemm(type, wp, (const float *)x, (float *)y, (int)rows, (int)cols, (int)batch,
                                         fits ? (void *)workspace : nullptr, fits ? workspace_bytes : 0, s));
-    for (size_t done = 0; done < batch; done += 8) {
-        const int n = (int)(batch - done < 8 ? batch - done : 8);
+    size_t n = 0;
+    for (size_t done = 0; done < batch; done += n) {
+        const size_t left = batch - done;
         const float *xp = (const float *)x + done * cols;
         float *yp = (float *)y + done * rows;
+        n = left < (size_t)kRowsTokens ? left : (size_t)kRowsTokens;
+        if (n > 8 && rows_tokens_supported(type, (int)rows, (int)cols, (int)n)) {
+            const int st = status(launch_rows_tokens(type, wp, xp, yp, (int)rows, (int)cols, (int)n, s));
+            if (st) return st;
+            continue;
+        }
+        n = left < 8 ? left : 8;
         if (dense) {
-            const int st = status(launch_dense(type, wp, xp, yp, (int)rows, (int)cols, n, s));
+            const int st = status(launch_dense(type, wp, xp, yp, (int)rows, (int)cols, (int)n, s));
             if (st) return st;
         } else if (n == 1) {
             const int st = status(launch_token(type, wp, xp, yp, (int)rows, (int)cols, s));
             if (st) return st;
-        } else if (smalln_rows_supported(type, (int)rows, (int)cols, n)) {
-            const int st = status(launch_smalln_rows(type, wp, xp, yp, (int)rows, (int)cols, n, s));
+        } else if (smalln_rows_supported(type, (int)rows, (int)cols, (int)n)) {
+            const int st = status(launch_smalln_rows(type, wp, xp, yp, (int)rows, (int)cols, (int)n, s));
             if (st) return st;
-        } else if ((fits && workspace_bytes >= smalln_workspace((int)cols, n))) {
-            const int st = status(launch_smalln(type, wp, xp, yp, (int)rows, (int)cols, n, (void *)workspace, s));
+        } else if ((fits && workspace_bytes >= smalln_workspace((int)cols, (int)n))) {
+            const int st = status(launch_smalln(type, wp, xp, yp, (int)rows, (int)cols, (int)n, (void *)workspace, s));
             if (st) return st;
         } else {
             // No room for the activation digits of several tokens: one at a time.
-            for (int k = 0; k < n; ++k) {
-                const int st = status(launch_token(type, wp, xp + (size_t)k * cols, yp + (size_t)k * rows,
+            for (size_t k = 0; k < n; ++k) {
+                const int st = status(launch_token(type, wp, xp + k * cols, yp + k * rows,
                                                    (int)rows, (int)cols, s));
                 if (st) return st;
             }
@@ -322,7 +328,8 @@ NYA_HIP_EXPORT const char *nya_hip_kernel_name(unsigned type, size_t rows, size_
         return dense_gemm_supported(type, (int)rows, (int)cols, (int)batch) ? "dense_gemm" : "skinny_dense";
     if (use_prefill(type, rows, cols, batch)) return prefill_kernel(type);
     if (batch == 1 && matvec_supported(type, (int)rows, (int)cols)) return matvec_kernel(type, (int)rows, (int)cols);
-    // Batches above 8 outside the GEMM run 8 tokens per launch.
+    // Batches above 8 outside the GEMM: rows of the same layout, many tokens or
+    // 8 per launch.
     const int n = batch < 8 ? (int)batch : 8;
     return smalln_rows_supported(type, (int)rows, (int)cols, n) ? "smalln_rows" : "smalln_mfma";
 }

@@ -89,6 +89,13 @@ bool smalln_rows_supported(unsigned type, int rows, int cols, int batch);
 hipError_t launch_smalln_rows(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
     int batch, hipStream_t stream);
 
+// Batches of 9..kRowsTokens of quantized weights in whole 256-column groups in
+// one launch without a workspace (rows_tokens.hip). x must be 16-byte aligned.
+constexpr int kRowsTokens = 64;
+bool rows_tokens_supported(unsigned type, int rows, int cols, int batch);
+hipError_t launch_rows_tokens(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
+    int batch, hipStream_t stream);
+
 // Activation digits of `batch` tokens x `cols` columns (row stride ldx) in
 // the layout of blockdot.h for np token slots (smalln.hip).
 hipError_t launch_quantize_x(const float *x, int ldx, int cols, int batch, int np, uint8_t *dig, float2 *meta,

@@ -138,3 +138,30 @@ def test_nonfinite_token(hip, t):
     assert np.array_equal(y[[0, 3]], clean[[0, 3]])
     for k in (1, 2):
         assert not np.isfinite(run(hip, w, t, rows, cols, x[k:k + 1], 1)).any()
+
+
+# Batches about the whole tiles of 16 tokens and the extra ones after them.
+MANY = [9, 16, 17, 18, 20, 21, 32, 33, 36, 37, 48, 49, 52, 53, 64]
+
+
+@pytest.mark.parametrize("t", QUANT, ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("rows,cols", [(40, 256), (16, 2048), (47, 2304), (1000, 4096), (130, 4864)],
+                         ids=["one-group", "half-tile", "ragged-rows", "many-rows", "uneven-groups"])
+def test_many_tokens_without_workspace(hip, oracle, t, rows, cols):
+    """Batches of 9..64 with no workspace on fp32 sums, against 64-bit sums of
+    the decoded weights: a weight is rounded once and a product's sum at most
+    64 times in its chain, then once per group and wavefront and 16 times at
+    the end: (84 + cols / 2048) 2^-24 of sum |w x|. Tokens of different
+    magnitudes and one with an infinity stay apart."""
+    w = synth.weights(t, rows, cols, 800 + t)
+    x = synth.activations(64, cols, 801 + t)
+    x *= np.float32(2.0) ** (np.arange(64, dtype=np.float32) % 7 * 9 - 27)[:, None]
+    exact, m = oracle.contract_sums(w, t, x, rows, cols)
+    for batch in MANY:
+        print(f"{TYPE_NAMES[t]} {rows}x{cols} batch {batch}", flush=True)
+        y = run(hip, w, t, rows, cols, x[:batch], batch, workspace=False)
+        assert np.all(np.abs(y - exact[:batch]) <= (84 + cols / 2048) * 2.0 ** -24 * m[:batch]), batch
+        bad = x[:batch].copy()
+        bad[batch - 1, cols - 1] = np.inf
+        z = run(hip, w, t, rows, cols, bad, batch, workspace=False)
+        assert np.array_equal(z[:-1], y[:-1]) and not np.isfinite(z[-1]).any()
