@@ -250,6 +250,9 @@ __device__ __forceinline__ void output_step(lds_u8 *__restrict__ kt, const lds_u
 // whose tiles fill the LDS.
 template <int W, int RG, int KS> constexpr int kPerSimd = W == 64 ? 2 : RG * KS / 4;
 
+// Workgroups of a shape that fits a CU twice, on the whole chip.
+template <int W, int RG> constexpr int kAtOnce = W == 64 && RG == 1 ? 512 : 0;
+
 template <int W, int RG, int KS>
 __global__ __launch_bounds__(64 * RG * KS)
 __attribute__((amdgpu_waves_per_eu(kPerSimd<W, RG, KS>, kPerSimd<W, RG, KS>))) void attention_tile(
@@ -264,8 +267,12 @@ __attribute__((amdgpu_waves_per_eu(kPerSimd<W, RG, KS>, kPerSimd<W, RG, KS>))) v
     const int rg = wave / KS, ks = wave % KS, h = lane >> 5;
     const int group = heads / kv_heads, rows = count * group;
     const int blocks = (rows + 32 * RG - 1) / (32 * RG);
-    // Later tokens see more: their workgroups start first.
-    const int kvh = blockIdx.x % kv_heads, block = blocks - 1 - (int)(blockIdx.x / kv_heads);
+    // Later tokens see more: their workgroups start first. Where all of them
+    // run at once, two to a CU, the second half of the grid goes from the first
+    // tokens on instead, so that a CU's two see about as many keys together.
+    const int kvh = blockIdx.x % kv_heads, b = (int)(blockIdx.x / kv_heads);
+    const int block = kAtOnce<W, RG> && (int)gridDim.x <= kAtOnce<W, RG> && 2 * b >= blocks ? b - (blocks + 1) / 2
+                                                                                          : blocks - 1 - b;
     const int row_raw = 32 * (RG * block + rg) + (lane & 31);
     const int row = row_raw < rows ? row_raw : rows - 1;
     const int token = row / group, head = kvh * group + row % group;
@@ -405,8 +412,13 @@ hipError_t launch_attention_tile(const float *q, int q_stride, const float *keys
     // Two row tiles per workgroup (a K and V tile read once for both) where
     // those workgroups fill the 256 CUs, else one (twice the
     // workgroups): 32 heads of 128 over 4096 positions, 256 tokens with one
-    // take 229 us, 512 tokens with two 368.
-    const bool pairs = (rows + 63) / 64 * kv_heads >= 256;
+    // take 229 us, 512 tokens with two 368. At width 64 two workgroups of one
+    // tile fit a CU: until those fill the chip, which the order of the grid
+    // balances (32/4 heads, 512 tokens from position 0: 33.5 us with two tiles,
+    // 26.7 with one; 16/16, 1024 tokens: 54 and 41; at positions 3584..4095 of
+    // 32/8 heads, where all see as much: 194 and 198; past one round the pairs
+    // win, 32/4 heads, 1024 tokens: 73 and 79).
+    const bool pairs = width == 64 ? (rows + 31) / 32 * kv_heads > kAtOnce<64, 1> : (rows + 63) / 64 * kv_heads >= 256;
 #define FY_TILE(WW, RGG, KSS) \
     launch_tile<WW, RGG, KSS>(q, q_stride, keys, values, out, positions, count, heads, kv_heads, max_length, window, scale, s)
     if (width == 64) return pairs ? FY_TILE(64, 2, 4) : FY_TILE(64, 1, 4);

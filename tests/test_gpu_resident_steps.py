@@ -346,7 +346,9 @@ def test_attention_ignores_rows_past_the_range(env, heads, kv_heads, width, leng
 RUN_CASES = [  # heads, kv_heads, width, max_length, count, first, window: count * heads past the tile kernel's threshold
     (32, 8, 128, 300, 64, 0, 0), (32, 8, 128, 700, 70, 601, 0), (32, 4, 64, 129, 65, 64, 0), (24, 8, 128, 250, 100, 33, 0),
     (32, 32, 128, 97, 97, 0, 40), (32, 1, 64, 200, 64, 130, 0), (32, 8, 128, 600, 513, 40, 64), (16, 8, 256, 300, 257, 17, 0),
-    (16, 8, 256, 400, 256, 140, 100), (8, 2, 128, 8300, 257, 8000, 0), (64, 8, 256, 600, 512, 80, 0)]
+    (16, 8, 256, 400, 256, 140, 100), (8, 2, 128, 8300, 257, 8000, 0), (64, 8, 256, 600, 512, 80, 0),
+    # Width 64 about the last grid of one row tile per workgroup, odd and even tile counts.
+    (32, 4, 64, 600, 512, 20, 0), (32, 4, 64, 560, 513, 20, 0), (16, 16, 64, 400, 300, 0, 0), (32, 8, 64, 300, 250, 9, 0)]
 
 
 @pytest.mark.parametrize("heads,kv_heads,width,max_length,count,first,window", RUN_CASES,
