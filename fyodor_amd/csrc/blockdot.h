@@ -1,6 +1,6 @@
-// Block dot products on gfx950 int8 MFMA, shared by the small-N path
-// (smalln.hip) and the prefill GEMM (prefill.hip): activation digits, the
-// tiled weight stages of one 256-column group, and the digit recombination.
+// Block dot products on gfx950 int8 MFMA of the small-N path (smalln.hip):
+// activation digits, the tiled weight stages of one 256-column group, and the
+// digit recombination. The other kernels over tiled weights use its types.
 //
 // Activations. Each 32-column group of a token's x is scaled by 2^(22-e)
 // (2^(e-1) <= max |x| < 2^e over the group) and rounded to integers X with

@@ -172,7 +172,7 @@ __device__ __forceinline__ void copy_group(lds_u8 *__restrict__ buf, const Piece
 {
     constexpr int kPairs = 16 * TW / RT;   // token pairs per wavefront, over all token tiles
     static_assert(kPairs >= 1 && 16 * TW % RT == 0, "whole token pairs per wavefront");
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % RT;
     const int vpair = 2 * ((lane & 1) * cols + 8 * (lane >> 1));   // bytes within the pair's two rows
 #pragma unroll
     for (int piece = 0; piece < 2; ++piece)
@@ -295,7 +295,7 @@ __device__ __forceinline__ void load_stage(WStage<T> &w, __amdgpu_buffer_rsrc_t 
 // with another count of loads in flight. The two buffers come in as restrict
 // pointers, which lets the compiler see that this step's LDS reads do not
 // depend on the copies it issues.
-template <unsigned T, int RT, int TW>
+template <unsigned T, int RT, int TW, int KS>
 __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], lds_u8 *__restrict__ buf,
     lds_u8 *__restrict__ nbuf, const Pieces &p, const Lane &L, __amdgpu_buffer_rsrc_t rs, int a_off, int cols, int m0,
     int g, int groups)
@@ -307,7 +307,7 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
     constexpr int kWaitCopies = (kLoads & 15) | ((kLoads >> 4) << 14) | (7 << 4) | (15 << 8);
     static_assert(kLoads < 64, "vmcnt field");
     const int lane = threadIdx.x & 63;
-    copy_group<RT, TW>(nbuf, p, cols, m0, g + 1 < groups ? g + 1 : g, sums);
+    copy_group<RT, TW>(nbuf, p, cols, m0, g + KS < groups ? g + KS : groups - 1, sums);
     // The weight loads below stay after the copies, in the compiler's view of
     // memory (the fence; the weights are not a restrict pointer) and in the
     // schedule.
@@ -385,6 +385,7 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
         for (int tt = 0; tt < TW; ++tt) {
             const h8 ys = *(const h8 *)(buf + kTileBytes * tt + 2 * kPieceBytes + 16 * lane);
             const f32x16 M = __builtin_amdgcn_mfma_f32_32x32x16_f16(ys, bm, (f32x16){}, 0, 0, 0);
+            if (KS > 1 && g >= groups) continue;   // the last group again, for the barriers
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[tt][r] = __builtin_fmaf(d, C[tt][r], __builtin_fmaf(ndmin, M[r], acc[tt][r]));
         }
@@ -420,7 +421,7 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
         if (group_blocks(L, g) == 8) blocks(std::true_type{});
         else blocks(std::false_type{});
     }
-    load_stage<T>(cur, rs, L, g + 2 < groups ? g + 2 : groups - 1);
+    load_stage<T>(cur, rs, L, g + 2 * KS < groups ? g + 2 * KS : groups - 1);
     // This wavefront's copies are complete; then every wavefront's are,
     // past the barrier. (The fence keeps the loads above before the wait.)
     asm volatile("" ::: "memory");
@@ -435,16 +436,23 @@ __device__ __forceinline__ void group_step(WStage<T> &cur, f32x16 (&acc)[TW], ld
 // of LDS, one workgroup per CU, 8 wavefronts of up to 256 VGPRs.
 // The weights are deliberately not a restrict pointer: the compiler may
 // then not move their loads across the memory fences of group_step.
-template <unsigned T, int RT, int TW>
-__global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1 ? RT / 2 : RT / 4, TW == 1 ? RT / 2 : RT / 4))) void prefill_f16(
+//
+// KS = 2 (Q4_K, RT = 4, TW = 1; launch_prefill_f16 says where): two sets of RT wavefronts take every other
+// group, each with buffers of its own, and the sums meet in LDS: two wavefronts
+// per SIMD where the grid gives a CU one workgroup.
+template <int RT, int TW, int KS> constexpr int kPerSimd = TW == 1 && KS == 1 ? RT / 2 : RT * KS / 4;
+template <unsigned T, int RT, int TW, int KS>
+__global__ __launch_bounds__(64 * RT * KS) __attribute__((amdgpu_waves_per_eu(kPerSimd<RT, TW, KS>, kPerSimd<RT, TW, KS>))) void prefill_f16(
     const uint8_t *w, Pieces p, float *__restrict__ y, int rows, int cols, int batch, int token_blocks)
 {
-    __shared__ __align__(16) uint8_t smem0[kBufBytes<TW>], smem1[kBufBytes<TW>];
-    lds_u8 *const B0 = (lds_u8 *)smem0, *const B1 = (lds_u8 *)smem1;
+    static_assert(KS == 1 || (T == Q4_K && TW == 1), "Q4_K, one token tile");
+    __shared__ __align__(16) uint8_t smem0[KS][kBufBytes<TW>], smem1[KS][kBufBytes<TW>];
+    const int ks = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / RT;
+    lds_u8 *const B0 = (lds_u8 *)smem0[ks], *const B1 = (lds_u8 *)smem1[ks];
     constexpr bool sums = T == Q4_K;
     // The wavefront index is uniform: keeping it scalar keeps the tile base
     // and the copy addresses in SGPRs.
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % RT;
     const int tiles = (rows + kTileRows - 1) / kTileRows;
     const int by = blockIdx.x % token_blocks, bx = blockIdx.x / token_blocks;
     const int tile_raw = RT * bx + wave;
@@ -470,10 +478,10 @@ __global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1
     // the compiler waits for all vector memory, those copies included, before
     // the first use of a register still loading; later steps read stages
     // completed by an earlier step's wait).
-    copy_group<RT, TW>(B0, p, cols, m0, 0, sums);
+    copy_group<RT, TW>(B0, p, cols, m0, ks < groups ? ks : groups - 1, sums);
     asm volatile("" ::: "memory");
-    load_stage<T>(st[0], rs, L, 0);
-    load_stage<T>(st[1], rs, L, groups > 1 ? 1 : 0);
+    load_stage<T>(st[0], rs, L, ks < groups ? ks : groups - 1);
+    load_stage<T>(st[1], rs, L, ks + KS < groups ? ks + KS : groups - 1);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0);
     barrier();
@@ -489,12 +497,26 @@ __global__ __launch_bounds__(64 * RT) __attribute__((amdgpu_waves_per_eu(TW == 1
     // merge a path on which stage 0's loads are still in flight, and the
     // compiler would wait for every load (the next group's copies included)
     // before each first step.
-    int g = 0;
-    for (; g + 1 < groups; g += 2) {
-        group_step<T, RT, TW>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
-        group_step<T, RT, TW>(st[1], acc, B1, B0, p, L, rs, a_off, cols, m0, g + 1, groups);
+    const int steps = (groups + KS - 1) / KS;
+    int i = 0;
+    for (; i + 1 < steps; i += 2) {
+        group_step<T, RT, TW, KS>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, ks + KS * i, groups);
+        group_step<T, RT, TW, KS>(st[1], acc, B1, B0, p, L, rs, a_off, cols, m0, ks + KS * (i + 1), groups);
     }
-    if (g < groups) group_step<T, RT, TW>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, g, groups);
+    if (i < steps) group_step<T, RT, TW, KS>(st[0], acc, B0, B1, p, L, rs, a_off, cols, m0, ks + KS * i, groups);
+    if constexpr (KS == 2) {
+        // (Every copy has landed: the last step's wait and barrier.)
+        float *const meet = (float *)&smem0[0][0] + 1024 * wave + lane;
+        static_assert(4096 * RT <= 2 * kBufBytes<TW>, "the sums fit the buffers");
+        if (ks == 1) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) meet[64 * r] = acc[0][r];
+        }
+        __syncthreads();
+        if (ks == 1) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][r] += meet[64 * r];
+    }
 
     if (tile_raw >= tiles || (lane & 31) >= R) return;
     const int row = kTileRows * tile + (lane & 31);
@@ -553,23 +575,30 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
     // One token tile: Q8_0/Q4_0 stages (16 loads) do not fit 128 VGPRs
     // without spilling: four-wavefront workgroups only.
     const bool wide = type == Q4_K && (tiles + 7) / 8 * tb >= 256;
+    // Q4_K where every workgroup has a CU to itself: two sets of wavefronts
+    // over the groups, us before and now: 14336 x 4096 x24 31.6, 28.1; 4096 x
+    // 4096 x64 28.5, 26.1; 4096 x 14336 x40 92.7, 77.9; 2048 x 2048 x512 22.0,
+    // 21.8. With more workgroups than CUs two of the single kind share one
+    // (2560 x 2048 x512 28.9, 33.2 split; 6144 x 4096 x256 49.7, 58.6).
+    const bool split = (long)(tiles + 3) / 4 * tb <= 256;
     const dim3 grid2((unsigned)((tiles + 7) / 8 * tb2));
     const dim3 grid((unsigned)((tiles + (wide ? 7 : 3)) / (wide ? 8 : 4) * tb));
-#define FY_PREFILL(TT, RTT, TWW, G, TB) \
-    hipLaunchKernelGGL((prefill_f16<TT, RTT, TWW>), G, dim3(64 * RTT), 0, s, w, p, y, rows, cols, batch, TB)
+#define FY_PREFILL(TT, RTT, TWW, KSS, G, TB) \
+    hipLaunchKernelGGL((prefill_f16<TT, RTT, TWW, KSS>), G, dim3(64 * RTT * KSS), 0, s, w, p, y, rows, cols, batch, TB)
     switch (type) {
     case Q4_K:
-        if (pair) FY_PREFILL(Q4_K, 8, 2, grid2, tb2);
-        else if (wide) FY_PREFILL(Q4_K, 8, 1, grid, tb);
-        else FY_PREFILL(Q4_K, 4, 1, grid, tb);
+        if (pair) FY_PREFILL(Q4_K, 8, 2, 1, grid2, tb2);
+        else if (wide) FY_PREFILL(Q4_K, 8, 1, 1, grid, tb);
+        else if (split) FY_PREFILL(Q4_K, 4, 1, 2, grid, tb);
+        else FY_PREFILL(Q4_K, 4, 1, 1, grid, tb);
         break;
     case Q8_0:
-        if (pair) FY_PREFILL(Q8_0, 8, 2, grid2, tb2);
-        else FY_PREFILL(Q8_0, 4, 1, grid, tb);
+        if (pair) FY_PREFILL(Q8_0, 8, 2, 1, grid2, tb2);
+        else FY_PREFILL(Q8_0, 4, 1, 1, grid, tb);
         break;
     case Q4_0:
-        if (pair) FY_PREFILL(Q4_0, 8, 2, grid2, tb2);
-        else FY_PREFILL(Q4_0, 4, 1, grid, tb);
+        if (pair) FY_PREFILL(Q4_0, 8, 2, 1, grid2, tb2);
+        else FY_PREFILL(Q4_0, 4, 1, 1, grid, tb);
         break;
     default: return hipErrorInvalidValue;
     }

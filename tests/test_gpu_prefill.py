@@ -61,7 +61,8 @@ def test_batch_and_row_tails(compute, oracle, type_id, batch):
 
 
 # One shape per workgroup form of the whole-group GEMM, with ragged rows and
-# tokens and group counts around the four-step rotation of the narrow forms
+# tokens and group counts around the four-step rotation of the narrow forms and
+# the two sets of wavefronts that take every other group (Q4_K, small grids)
 # (rows, cols, batch): 64 x 32, 128 x 32, 128 x 64, 256 x 64.
 TILE_FORMS = [(200, 256, 33), (75, 512, 40), (300, 768, 65), (33, 1280, 97), (2081, 1024, 513), (4097, 512, 161),
               (4000, 1280, 129), (8161, 256, 200), (8161, 768, 200), (16100, 512, 300), (33001, 256, 170)]
