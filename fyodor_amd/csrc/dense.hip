@@ -247,10 +247,16 @@ __device__ __forceinline__ void store_tokens(const float (&x)[16], int half, uin
 
 // Slice s in pieces; big becomes the largest magnitude met (a BF16 pair's
 // second value is taken with the first one's bits below it; F16 stays below
-// the 2^16 that big starts from).
+// the 2^16 that big starts from), seen the bits of all weights together.
 template <unsigned T>
-__device__ __forceinline__ void weight_pieces(const GemmWeights<T> &st, int s, bf16x8 (&out)[kPieces<T>], float &big)
+__device__ __forceinline__ void weight_pieces(const GemmWeights<T> &st, int s, bf16x8 (&out)[kPieces<T>], float &big,
+    uint32_t &seen)
 {
+    constexpr int kWords = T == F32 ? 2 : 1;
+#pragma unroll
+    for (int q = 0; q < kWords; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) seen |= st.w[kWords * s + q][i];
     if constexpr (T == BF16) {
         out[0] = __builtin_bit_cast(bf16x8, st.w[s]);
 #pragma unroll
@@ -279,6 +285,13 @@ __device__ __forceinline__ void weight_pieces(const GemmWeights<T> &st, int s, b
     }
 }
 
+template <unsigned T>
+__device__ __forceinline__ float weight_at(const uint8_t *w, size_t at)
+{
+    if constexpr (T == F32) return ((const float *)w)[at];
+    else return widen<T>(((const uint16_t *)w)[at]);
+}
+
 // One output as a plain fp32 dot over columns [k0, k1), by the wavefront.
 template <unsigned T>
 __device__ float plain_dot(const uint8_t *w, const float *x, int cols, int row, int token, int k0, int k1)
@@ -286,13 +299,7 @@ __device__ float plain_dot(const uint8_t *w, const float *x, int cols, int row, 
     const float *xr = x + (size_t)token * cols;
     float s = 0.f;
 #pragma unroll 8
-    for (int k = k0 + (int)(threadIdx.x & 63); k < k1; k += 64) {
-        const size_t at = (size_t)row * cols + k;
-        float wv;
-        if constexpr (T == F32) wv = ((const float *)w)[at];
-        else wv = widen<T>(((const uint16_t *)w)[at]);
-        s += wv * xr[k];
-    }
+    for (int k = k0 + (int)(threadIdx.x & 63); k < k1; k += 64) s += weight_at<T>(w, (size_t)row * cols + k) * xr[k];
     return wave_sum(s);
 }
 
@@ -326,6 +333,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // step i - 1, are split into the other buffer, and those of step i + 2
     // requested.
     float big = T == F16 ? 0x1p16f : 0.f;   // the largest |w| and |x| met
+    uint32_t seen = 0;                      // the bits of this lane's weights
     GemmWeights<T> w0, w1;
     float x0[16], x1[16];
     auto at = [&](int i) { return first + i * kGemmK; };
@@ -343,7 +351,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int p = 0; p < 3; ++p)
                     x8[t][p] = *(const bf16x8 *)(buf + p * kPlaneBytes + 128 * (32 * t + (lane & 31)) +
                                                  16 * ((2 * s + h) ^ ((lane >> 1) & 7)));
-            weight_pieces<T>(cur, s, w8, big);
+            weight_pieces<T>(cur, s, w8, big, seen);
         };
         // A slice's operands are made among the MFMAs of the one before, but
         // for F32, whose second set would not fit the registers.
@@ -403,9 +411,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // The halves meet in LDS. D[token][row]: register i of lane l holds token
     // 8 (i / 4) + 4 h + i % 4 of its token tile, row l % 32.
     float *meet = (float *)&sx[0][0][0] + 2048 * wr + lane, *most = (float *)&sx[0][0][0] + 8192;
+    uint32_t *bits = (uint32_t *)most + 8 + 64 * wr + lane;
     for (int o = 32; o; o >>= 1) big = __builtin_fmaxf(big, __shfl_xor(big, o, 64));
     if (lane == 0) most[wave] = big;
     if (ks == 1) {
+        *bits = seen;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -418,27 +428,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float least = (float)cols * 0x1p-99f * big;
     float *out = gridDim.z == 1 ? y : part + (size_t)blockIdx.z * batch * rows;
     auto token = [&](int i) { return t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3); };
-    uint32_t again = 0;
+    uint32_t again = 0, zero = 0;
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
         const float v = (acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15]) + meet[64 * i];
         if (row < rows && token(i) < batch) {
             const float m = __builtin_fabsf(v);
             if (!(m >= least && m <= 3.402823466e38f)) again |= 1u << i;
+            if (m == 0.f) zero |= 1u << i;
             out[(size_t)token(i) * rows + row] = v;
         }
     }
     if (__ballot(again != 0) == 0) return;
+    // The zeros of a row of zeros stand.
+    seen |= *bits;
+    seen |= (uint32_t)__shfl_xor((int)seen, 32, 64);
+    if ((seen & (T == F32 ? 0x7FFFFFFFu : 0x7FFF7FFFu)) == 0) again &= ~zero;
     for (int i = 0; i < 32; ++i)
         for (int half = 0; half < 2; ++half) {
             uint64_t need = __ballot(again >> i & 1) & 0xFFFFFFFFull << 32 * half;
             if (need == 0) continue;
             const int tok = __builtin_amdgcn_readlane(token(i), 32 * half);
-            // The zeros of a token of zeros stand.
+            // So do those of a token of zeros.
             bool any = false;
 #pragma unroll 16
             for (int k = k0 + lane; k < k1; k += 64) any |= x[(size_t)tok * cols + k] != 0.f;
-            if (__ballot(any) == 0) need = __ballot((again >> i & 1) && out[(size_t)tok * rows + row] != 0.f) & need;
+            if (__ballot(any) == 0) need &= ~__ballot(zero >> i & 1);
             while (need) {
                 const int l = __ffsll((unsigned long long)need) - 1, at = __builtin_amdgcn_readlane(row, l);
                 need &= need - 1;
@@ -462,10 +477,11 @@ __global__ __launch_bounds__(256) void dense_combine(const float *__restrict__ p
 // us before (one fp32 MFMA chain, 64 x 64 tiles) and now, 4096 x 4096 by
 // tokens, alone on the stream:
 //          16          333          512          2048
-//   F16    38 -> 18    219 -> 70    235 -> 83    690 -> 335
-//   BF16   38 -> 18    243 -> 64    241 -> 67
-//   F32    34 -> 28    208 -> 112   213 -> 115
-// At 512 tokens that is 1030 (F16), 770 (BF16) and 900 (F32) TFLOP/s issued
+//   F16    38 -> 19    219 -> 70    235 -> 85    690 -> 345
+//   BF16   38 -> 18    243 -> 68    241 -> 71
+//   F32    34 -> 28    208 -> 105   213 -> 115
+// (of which the largest magnitude and the rows' bits cost 3 to 5 us at 512.)
+// At 512 tokens that is 1010 (F16), 730 (BF16) and 900 (F32) TFLOP/s issued
 // of the 1406 a large bf16 product reaches here: what bounds it now. Rows of
 // a multiple of 16 bytes load 16 bytes per lane; the others element by
 // element (F32 300 x 1002, 300 tokens: 39 -> 16.5 us).

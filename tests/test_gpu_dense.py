@@ -150,6 +150,7 @@ def test_dense_gemm_non_finite(hip, t):
     wv[3, 199], wv[64, 0], wv[129, 100], wv[7, 50], wv[7, 51] = np.inf, -np.inf, np.nan, np.inf, np.inf
     x[0, 64], x[9, 199], x[63, 5], x[69, 150] = np.inf, 0.0, -np.inf, np.nan
     x[20], x[30], x[40:48] = 0.0, 1e-40, 0.0
+    wv[32], wv[60:63], wv[128] = 0.0, 0.0, 0.0
     x[20, 3], x[21, 4] = np.float32(3.4028235e38), np.float32(-3.4e38)
     w, wv = stored(t, wv)
     with np.errstate(invalid="ignore"):
