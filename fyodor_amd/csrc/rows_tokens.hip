@@ -340,6 +340,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
             for (int e = 0; e < EXTRA; ++e) acc.more[e] += part.more[e];
         }
+        // Copies requested ahead are still in flight into these buffers, which
+        // past the barrier hold other wavefronts' sums.
+        wait_loads<0>();
     }
     __syncthreads();
     float *const red = (float *)lds;   // [wave][share][lane]
