@@ -165,10 +165,13 @@ __device__ __forceinline__ void output_tile(const lds_u8 *vt, const QueryRow &qr
     const float next = fmaxf(m, top);
     const float alpha = next == m ? 1.f : expf(m - next);
     m = next;
+    // Scores of minus infinity have probability 0 also where the row has seen
+    // nothing else yet (a row that never does ends in 0 / 0).
+    const float top_seen = next == -INFINITY ? 0.f : next;
     float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        float e = expf(S[i] - next);
+        float e = expf(S[i] - top_seen);
         if constexpr (BOUNDARY) {
             if (from + (unsigned)(8 * (i >> 2) + (i & 3)) >= span) e = 0.f;
         }

@@ -408,6 +408,44 @@ def test_attention_runs(env, heads, kv_heads, width, max_length, count, first, w
             assert np.all(np.isfinite(got[i])) != sees[i]
 
 
+@pytest.mark.parametrize("heads,kv_heads,width,count,first,window",
+                         [(32, 8, 128, 128, 0, 0), (32, 4, 64, 160, 70, 0), (16, 8, 256, 512, 0, 0), (32, 8, 128, 200, 30, 50)],
+                         ids=["128", "64", "256", "window"])
+def test_attention_runs_infinite_scores(env, heads, kv_heads, width, count, first, window):
+    """Scores of minus infinity weigh nothing: one key, the last that some
+    token sees and so its key tile's only seen one, a whole tile of keys, and a
+    range of several tiles. Only the tokens that see nothing else give NaN
+    (0 / 0, as the maximum over all keys gives them)."""
+    rt, L, stream = env
+    rng = np.random.default_rng(width + count + window)
+    n = first + count
+    q = rng.standard_normal((count, heads * width)).astype(np.float32)
+    q[:, ::width] = np.abs(q[:, ::width]) + 1
+    keys = rng.standard_normal((n, kv_heads * width)).astype(np.float32)
+    values = rng.standard_normal((n, kv_heads * width)).astype(np.float32)
+    hidden = [0, 32, 33, 64] + list(range(96, 128)) + list(range(first + 2, first + 12))
+    keys[hidden, ::width] = -np.inf
+    positions = np.arange(first, n, dtype=np.int32)
+    scale = float(1 / np.sqrt(np.float32(width)))
+    dev = Dev(rt)
+    try:
+        qd, kd, vd, pd = dev.put(q), dev.put(keys), dev.put(values), dev.put(positions)
+        od = dev.put(np.full((count, heads * width), 7.0, np.float32))
+        print(f"infinite scores {heads}/{kv_heads} x {width}, {count} from {first}, window {window}", flush=True)
+        assert L.nya_hip_attention(qd, heads * width, kd, vd, od, 0, pd, count, heads, kv_heads, width, n, window, scale,
+                                   stream) == 0
+        rt.sync(stream)
+        got = dev.get(od, np.empty((count, heads * width), np.float32))
+    finally:
+        dev.close()
+    with np.errstate(invalid="ignore"):
+        ref = np.stack([attention_ref(q[i], keys, values, heads, kv_heads, width, first + i + 1, np.float32(scale), window)
+                        for i in range(count)])
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    good = ~np.isnan(ref)
+    assert scaled_error(got[good], ref[good]) <= 2e-6
+
+
 SPLIT_CASES = [(32, 8, 128, 4096, 1, 64, 0), (32, 4, 64, 1000, 1, 16, 0), (8, 8, 128, 300, 1, 8, 0),
                (16, 8, 128, 2000, 3, 32, 0), (8, 2, 256, 5000, 2, 8, 0), (32, 4, 64, 20000, 1, 32, 0),
                (32, 8, 128, 5, 1, 64, 0), (32, 8, 128, 257, 33, 8, 0), (8, 2, 128, 600, 2, 300, 0),
