@@ -211,15 +211,21 @@ __device__ __forceinline__ void output_tile(const lds_u8 *vt, const QueryRow &qr
         if constexpr (BOUNDARY) {
             if (__builtin_amdgcn_ballot_w64(odd)) {
                 // Rare: this lane's columns 64 part + 2 x + e, x = 8 (i / 4) + 4 h + i % 4.
+                // `none`: the row's keys of probability 0.
+                uint32_t none = 0;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) none |= (S[i] == 0.f ? 1u : 0u) << (8 * (i >> 2) + 4 * h + (i & 3));
+                none |= (uint32_t)__shfl_xor((int)none, 32, 64);
 #pragma unroll 1
                 for (int t = 0; t < kKeys; ++t) {
                     const bool seen = key0 + t >= qr.first && key0 + t <= qr.last;
+                    const float p = none >> t & 1 ? 0.f : 1.f;   // (not finite times more than 0: itself)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const float2 v = *(const float2 *)(vt + 4 * W * t + 256 * part +
                                                            8 * (8 * (i >> 2) + 4 * h + (i & 3)));
-                        if (seen && !finite_bits(v.x)) t0[i] += v.x;
-                        if (seen && !finite_bits(v.y)) t1[i] += v.y;
+                        if (seen && !finite_bits(v.x)) t0[i] += v.x * p;
+                        if (seen && !finite_bits(v.y)) t1[i] += v.y * p;
                     }
                 }
             }

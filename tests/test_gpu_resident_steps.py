@@ -415,7 +415,10 @@ def test_attention_runs_infinite_scores(env, heads, kv_heads, width, count, firs
     """Scores of minus infinity weigh nothing: one key, the last that some
     token sees and so its key tile's only seen one, a whole tile of keys, and a
     range of several tiles. Only the tokens that see nothing else give NaN
-    (0 / 0, as the maximum over all keys gives them)."""
+    (0 / 0, as the maximum over all keys gives them). An infinite value of such
+    a key leaves NaN (0 times infinity) in its column of the tokens that see
+    the key, whole key tiles or part of one, and infinity beside a probability
+    above 0."""
     rt, L, stream = env
     rng = np.random.default_rng(width + count + window)
     n = first + count
@@ -425,6 +428,8 @@ def test_attention_runs_infinite_scores(env, heads, kv_heads, width, count, firs
     values = rng.standard_normal((n, kv_heads * width)).astype(np.float32)
     hidden = [0, 32, 33, 64] + list(range(96, 128)) + list(range(first + 2, first + 12))
     keys[hidden, ::width] = -np.inf
+    values[33, 3], values[100, width - 1], values[first + 5, 2] = np.inf, -np.inf, np.inf
+    values[first + 20, 9], values[first + 21, 10] = np.inf, -np.inf
     positions = np.arange(first, n, dtype=np.int32)
     scale = float(1 / np.sqrt(np.float32(width)))
     dev = Dev(rt)
@@ -442,7 +447,8 @@ def test_attention_runs_infinite_scores(env, heads, kv_heads, width, count, firs
         ref = np.stack([attention_ref(q[i], keys, values, heads, kv_heads, width, first + i + 1, np.float32(scale), window)
                         for i in range(count)])
     assert np.array_equal(np.isnan(got), np.isnan(ref))
-    good = ~np.isnan(ref)
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.all(got[np.isinf(ref)] == ref[np.isinf(ref)])
+    good = np.isfinite(ref)
     assert scaled_error(got[good], ref[good]) <= 2e-6
 
 
