@@ -68,8 +68,10 @@ hipError_t launch_token(unsigned type, const uint8_t *w, const float *x, float *
     return launch_smalln(type, w, x, y, rows, cols, 1, nullptr, s);
 }
 
+// `whole`: the tokens of the caller's call, of which these are `batch`: it
+// decides the route and the kernel's form (launch_prefill).
 int matmul_impl(uintptr_t w, unsigned type, size_t rows, size_t cols, uintptr_t x, uintptr_t y, size_t batch,
-    uintptr_t workspace, size_t workspace_bytes, uintptr_t stream)
+    size_t whole, uintptr_t workspace, size_t workspace_bytes, uintptr_t stream)
 {
     size_t b;
     if (!w || !x || !y || !batch || batch > INT_MAX || !storage_bytes(type, rows, cols, &b)) return 1;
@@ -81,9 +83,9 @@ int matmul_impl(uintptr_t w, unsigned type, size_t rows, size_t cols, uintptr_t 
     const bool fits = workspace && !(workspace & 15u);
     // The GEMM needs its workspace; without one (or a short one) the batch is
     // run up to 64 or 8 columns at a time instead.
-    if (use_prefill(type, rows, cols, batch) && fits && workspace_bytes >= prefill_workspace(type, (int)cols, (int)batch))
+    if (use_prefill(type, rows, cols, whole) && fits && workspace_bytes >= prefill_workspace(type, (int)cols, (int)batch))
         return status(launch_prefill(type, wp, (const float *)x, (float *)y, (int)rows, (int)cols, (int)batch,
-                                     (void *)workspace, s));
+                                     (int)whole, (void *)workspace, s));
     if (dense && dense_gemm_supported(type, (int)rows, (int)cols, (int)batch))
         return status(launch_dense_gemm(type, wp, (const float *)x, (float *)y, (int)rows, (int)cols, (int)batch,
                                         fits ? (void *)workspace : nullptr, fits ? workspace_bytes : 0, s));
@@ -209,7 +211,7 @@ NYA_HIP_EXPORT int nya_hip_workspace_bytes(unsigned type, size_t rows, size_t co
 NYA_HIP_EXPORT int nya_hip_matmul(uintptr_t w, unsigned type, size_t rows, size_t cols,
     uintptr_t x, uintptr_t y, size_t batch, uintptr_t workspace, size_t workspace_bytes, uintptr_t stream)
 {
-    return matmul_impl(w, type, rows, cols, x, y, batch, workspace, workspace_bytes, stream);
+    return matmul_impl(w, type, rows, cols, x, y, batch, batch, workspace, workspace_bytes, stream);
 }
 
 NYA_HIP_EXPORT int nya_hip_matmul_static(uintptr_t w, unsigned type, size_t rows, size_t cols, uintptr_t x,
@@ -222,24 +224,26 @@ NYA_HIP_EXPORT int nya_hip_matmul_static(uintptr_t w, unsigned type, size_t rows
     if (!ws) return -(int)hipErrorInvalidSymbol;
     // The prefill GEMM runs in token chunks whose workspace fits the array
     // (every token is independent of the others): `parts` chunks of nearly
-    // equal size, each above half the array's capacity (at least 32 tokens),
-    // so every chunk stays on the GEMM and every token gets the same result
-    // as through nya_hip_matmul. Where not even 64 tokens of the GEMM's
-    // workspace fit (rows of about 254k columns and more), the batch runs
-    // as 8-token launches, as nya_hip_matmul does with a short workspace.
+    // equal size, each in the form that the whole batch has, so every token
+    // gets the same result as through nya_hip_matmul. Where not even 64 tokens
+    // of the GEMM's workspace fit (rows of about 254k columns and more), the
+    // batch runs without the GEMM, as nya_hip_matmul does with a short
+    // workspace.
     // Every other path needs at most a few hundred KiB (the small-N digits
     // of one 16384-column chunk); matmul_impl itself falls back to launches
     // without scratch where even that would not fit.
     size_t parts = 1;
     if (use_prefill(type, rows, cols, batch)) {
         const size_t fit = static_chunk_tokens(type, cols);
-        if (fit < 64) return matmul_impl(w, type, rows, cols, x, y, batch, (uintptr_t)ws, kStaticScratchBytes, stream);
+        if (fit < 64)
+            return matmul_impl(w, type, rows, cols, x, y, batch, batch, (uintptr_t)ws, kStaticScratchBytes, stream);
         parts = (batch + fit - 1) / fit;
     }
     for (size_t part = 0, done = 0; part < parts; ++part) {
         const size_t n = batch / parts + (part < batch % parts ? 1 : 0);
         const int st = matmul_impl(w, type, rows, cols, x + done * cols * sizeof(float),
-                                   y + done * rows * sizeof(float), n, (uintptr_t)ws, kStaticScratchBytes, stream);
+                                   y + done * rows * sizeof(float), n, batch, (uintptr_t)ws, kStaticScratchBytes,
+                                   stream);
         if (st) return st;
         done += n;
     }

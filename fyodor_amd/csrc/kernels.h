@@ -104,23 +104,25 @@ hipError_t launch_quantize_x(const float *x, int ldx, int cols, int batch, int n
 // Batches above 8 with quantized weights, on fp16 MFMA (prefill.hip chooses
 // between prefill_tile.hip and prefill_f16.hip). The launch needs
 // prefill_workspace bytes of 16-byte-aligned device scratch; prefill_kernel
-// names the GEMM kernel.
+// names the GEMM kernel. `whole`: the tokens of the call that this batch is a
+// part of; it chooses the kernel and its form (they differ in the order of their
+// sums), so that a token's result does not depend on how a call was cut.
 size_t prefill_workspace(unsigned type, int cols, int batch);
 hipError_t launch_prefill(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
-    void *workspace, hipStream_t stream);
+    int whole, void *workspace, hipStream_t stream);
 const char *prefill_kernel(unsigned type);
 
 // Whole 256-column groups (prefill_tile.hip): every Q8_0, Q4_0 and Q6_K batch
 // of them, Q4_K batches that fill the chip. np: the tokens the workspace holds
 // pieces of (batch rounded up to a multiple of 32).
-bool prefill_tile_supported(unsigned type, int rows, int cols, int batch);
+bool prefill_tile_supported(unsigned type, int rows, int cols, int whole);
 hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
-    void *workspace, int np, hipStream_t s);
+    int whole, void *workspace, int np, hipStream_t s);
 // The other Q4_K batches, and Q8_0 / Q4_0 rows with a short last group
 // (prefill_f16.hip).
 size_t prefill_f16_workspace(int cols, int batch);
 hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
-    int batch, void *workspace, hipStream_t stream);
+    int batch, int whole, void *workspace, hipStream_t stream);
 
 // Dense F32 / F16 / BF16 batches above 8 as one GEMM on the fp32 matrix cores
 // (dense.hip).

@@ -18,12 +18,12 @@ size_t prefill_workspace(unsigned type, int cols, int batch)
 const char *prefill_kernel(unsigned type) { return type == Q6_K ? "prefill_mfma" : "prefill_f16"; }
 
 hipError_t launch_prefill(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
-    void *workspace, hipStream_t s)
+    int whole, void *workspace, hipStream_t s)
 {
     const int pad = type == Q6_K ? 32 : 64, np = (int)(((long)batch + pad - 1) / pad * pad);
-    if (prefill_tile_supported(type, rows, cols, batch))
-        return launch_prefill_tile(type, w, x, y, rows, cols, batch, workspace, np, s);
-    return launch_prefill_f16(type, w, x, y, rows, cols, batch, workspace, s);
+    if (prefill_tile_supported(type, rows, cols, whole))
+        return launch_prefill_tile(type, w, x, y, rows, cols, batch, whole, workspace, np, s);
+    return launch_prefill_f16(type, w, x, y, rows, cols, batch, whole, workspace, s);
 }
 
 }  // namespace fy

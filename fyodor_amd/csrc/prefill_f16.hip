@@ -559,7 +559,7 @@ size_t prefill_f16_workspace(int cols, int batch)
 }
 
 hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
-    int batch, void *workspace, hipStream_t s)
+    int batch, int whole, void *workspace, hipStream_t s)
 {
     const int np = (batch + 2 * kTokens - 1) / (2 * kTokens) * (2 * kTokens);
     const Pieces p = pieces_of(workspace, cols, np);
@@ -569,18 +569,18 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
     // Two token tiles per wavefront (each weight operand serves four MFMAs)
     // where one workgroup per CU of 256 rows x 64 tokens fills the chip (Q4_K
     // batches that do are prefill_tile.hip's).
-    const int tb2 = (batch + 2 * kTokens - 1) / (2 * kTokens);
-    const int tb = (batch + kTokens - 1) / kTokens;
-    const bool pair = (tiles + 7) / 8 * tb2 >= 256;
+    const int tb2 = (batch + 2 * kTokens - 1) / (2 * kTokens), whole2 = (whole + 2 * kTokens - 1) / (2 * kTokens);
+    const int tb = (batch + kTokens - 1) / kTokens, whole1 = (whole + kTokens - 1) / kTokens;
+    const bool pair = (long)(tiles + 7) / 8 * whole2 >= 256;
     // One token tile: Q8_0/Q4_0 stages (16 loads) do not fit 128 VGPRs
     // without spilling: four-wavefront workgroups only.
-    const bool wide = type == Q4_K && (tiles + 7) / 8 * tb >= 256;
+    const bool wide = type == Q4_K && (long)(tiles + 7) / 8 * whole1 >= 256;
     // Q4_K where every workgroup has a CU to itself: two sets of wavefronts
     // over the groups, us before and now: 14336 x 4096 x24 31.6, 28.1; 4096 x
     // 4096 x64 28.5, 26.1; 4096 x 14336 x40 92.7, 77.9; 2048 x 2048 x512 22.0,
     // 21.8. With more workgroups than CUs two of the single kind share one
     // (2560 x 2048 x512 28.9, 33.2 split; 6144 x 4096 x256 49.7, 58.6).
-    const bool split = (long)(tiles + 3) / 4 * tb <= 256;
+    const bool split = (long)(tiles + 3) / 4 * whole1 <= 256;
     const dim3 grid2((unsigned)((tiles + 7) / 8 * tb2));
     const dim3 grid((unsigned)((tiles + (wide ? 7 : 3)) / (wide ? 8 : 4) * tb));
 #define FY_PREFILL(TT, RTT, TWW, KSS, G, TB) \

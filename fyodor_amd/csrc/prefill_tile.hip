@@ -739,9 +739,9 @@ hipError_t launch_wide(unsigned type, const uint8_t *w, const Pieces &p, float *
 //   Q4_K 4096x4096  x512    105 /  69 /  65 /  70    48
 enum Shape { kRows64, kRows128, kRows128Wide, kRows256, kElsewhere };
 
-static Shape shape_of(unsigned type, int rows, int batch)
+static Shape shape_of(unsigned type, int rows, int whole)
 {
-    const long t32 = ((long)batch + 31) / 32, t64 = ((long)batch + 63) / 64;
+    const long t32 = ((long)whole + 31) / 32, t64 = ((long)whole + 63) / 64;
     auto blocks = [&](int per) { return ((long)rows + per - 1) / per; };
     if (type == Q4_K) return blocks(256) * t64 > 256 ? kRows256 : kElsewhere;
     if (blocks(64) * t32 <= 256) return kRows64;
@@ -750,18 +750,18 @@ static Shape shape_of(unsigned type, int rows, int batch)
     return kRows256;
 }
 
-bool prefill_tile_supported(unsigned type, int rows, int cols, int batch)
+bool prefill_tile_supported(unsigned type, int rows, int cols, int whole)
 {
-    return cols % kGroupCols == 0 && shape_of(type, rows, batch) != kElsewhere;
+    return cols % kGroupCols == 0 && shape_of(type, rows, whole) != kElsewhere;
 }
 
 hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
-    void *workspace, int np, hipStream_t s)
+    int whole, void *workspace, int np, hipStream_t s)
 {
     const Pieces p = pieces_of(workspace, cols, np);
     const hipError_t e = launch_split_x(x, batch, cols, p, true, s);
     if (e != hipSuccess) return e;
-    switch (shape_of(type, rows, batch)) {
+    switch (shape_of(type, rows, whole)) {
     case kRows64: return launch_blocks<1, 1>(type, w, p, y, rows, cols, batch, np, s);
     case kRows128: return launch_blocks<1, 2>(type, w, p, y, rows, cols, batch, np, s);
     case kRows128Wide: return launch_blocks<2, 2>(type, w, p, y, rows, cols, batch, np, s);

@@ -94,11 +94,11 @@ NYA_HIP_EXPORT int nya_hip_matmul(uintptr_t w, unsigned type, size_t rows, size_
  * scratch is a fixed device array of NYA_HIP_STATIC_SCRATCH_BYTES inside
  * this library, one per GPU, held until the process ends; the call
  * allocates and frees nothing. Prefill batches (above 8 tokens) run in
- * token chunks whose scratch fits the array; where not even a 64-token
- * chunk fits (rows of about 254k columns and more) the batch runs as
- * 8-token launches, which is what nya_hip_matmul does with a workspace
- * shorter than it asks for (then the results equal that call's, not the
- * GEMM's). Returns 0, 1 when declined (the rules of nya_hip_matmul), <0 on
+ * token chunks whose scratch fits the array, each in the kernel form that
+ * the whole batch has; where not even a 64-token chunk fits (rows of about
+ * 254k columns and more) the batch runs without the GEMM, which is what
+ * nya_hip_matmul does with a workspace shorter than it asks for (then the
+ * results equal that call's, not the GEMM's). Returns 0, 1 when declined (the rules of nya_hip_matmul), <0 on
  * a HIP failure; NYA_HIP_STATUS_SCRATCH is kept for callers that test for
  * it and is not returned. Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (other streams, other

@@ -6,7 +6,9 @@ smaller input, so the second reads a scratch array the first left full;
 the outputs must equal the workspace entry point's bit for bit (same
 kernels on the same tokens). Cases: the fp16 prefill GEMM in one chunk and
 in two (4096 x 14336 at 2048 tokens needs 121 MB of scratch against the
-array's 64 MiB), the int8 Q6_K prefill, the small-N tile kernel's digits
+array's 64 MiB; 1024 and 2048 rows, where the chunks alone would take a form
+with another order of sums than the whole batch, and 65 tokens of rows so wide
+that a chunk alone would not take the GEMM), Q6_K's GEMM, the small-N tile kernel's digits
 (the only batch of 2..8 that uses scratch) and the batch-1 matvec; and
 rows too wide for any GEMM chunk to fit the array.
 """
@@ -23,6 +25,10 @@ SCRATCH = 64 << 20
 CASES = [
     (Q4_K, 14336, 4096, (2048, 40)),
     (Q4_K, 4096, 14336, (2048, 100)),
+    (Q4_K, 1024, 14336, (2048, 100)),
+    (Q6_K, 2048, 14336, (2048, 60)),
+    (Q8_0, 4096, 14336, (1300, 40)),
+    (Q6_K, 256, 131072, (65, 40)),
     (Q6_K, 4096, 4096, (300, 20)),
     (Q4_K, 14336, 8192, (8, 3)),
     (Q8_0, 4096, 4096, (1, 1)),
