@@ -332,8 +332,9 @@ NYA_HIP_EXPORT const char *nya_hip_kernel_name(unsigned type, size_t rows, size_
         return dense_gemm_supported(type, (int)rows, (int)cols, (int)batch) ? "dense_gemm" : "skinny_dense";
     if (use_prefill(type, rows, cols, batch)) return prefill_kernel(type);
     if (batch == 1 && matvec_supported(type, (int)rows, (int)cols)) return matvec_kernel(type, (int)rows, (int)cols);
-    // Batches above 8 outside the GEMM: rows of the same layout, many tokens or
-    // 8 per launch.
+    // Batches above 8 outside the GEMM: up to 64 tokens per launch, or 8.
+    const int many = batch < (size_t)kRowsTokens ? (int)batch : kRowsTokens;
+    if (rows_tokens_supported(type, (int)rows, (int)cols, many)) return "rows_tokens";
     const int n = batch < 8 ? (int)batch : 8;
     return smalln_rows_supported(type, (int)rows, (int)cols, n) ? "smalln_rows" : "smalln_mfma";
 }

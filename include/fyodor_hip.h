@@ -80,8 +80,10 @@ NYA_HIP_EXPORT int nya_hip_workspace_bytes(unsigned type, size_t rows, size_t co
     size_t batch, size_t *bytes);
 
 /* Enqueue Y = X * W^T for batch >= 1 (replaces rocm/rocm.c:127-128).
- * batch 1 is the decode matvec, batch 2..8 the small-N path and larger
- * batches the prefill GEMM. `workspace` holds at least the bytes reported
+ * batch 1 is the decode matvec, batch 2..8 the small-N path, and larger
+ * batches run up to 64 tokens per launch without a workspace (small ones, and
+ * any whose workspace is missing or short; 8 per launch where that kernel does
+ * not take the shape) or on the prefill GEMM. `workspace` holds at least the bytes reported
  * by nya_hip_workspace_bytes for the same arguments (it may be 0 then). */
 NYA_HIP_EXPORT int nya_hip_matmul(uintptr_t w, unsigned type, size_t rows, size_t cols,
     uintptr_t x, uintptr_t y, size_t batch, uintptr_t workspace, size_t workspace_bytes,

@@ -201,12 +201,14 @@ def test_prefill_dispatch_and_workspace():
     """Batch 1 needs no workspace; batches of 2..8 need the activation digits
     of a padded token count; batches above 8 go to the prefill GEMM: fp16
     activation pieces for Q4_K/Q8_0/Q4_0 (per token, rounded up to 64
-    tokens: two fp16 planes, the 32-column block sums and the scale), int8
-    digits for Q6_K (rounded up to 32 tokens) -- except small batches of
-    matrices the row-balanced small-N kernel takes, which run 8 tokens per
-    launch up to a break-even batch (20 tokens from 8192 rows on, else 32;
-    Q6_K only on rows wider than 4096 columns, up to 56); dense types need
-    none, and run batches above 8 on their own GEMM (nothing is launched)."""
+    tokens: two fp16 planes, the 32-column block sums and the scale), and for
+    Q6_K in room for 136 bytes per 32 columns (rounded up to 32 tokens) --
+    except small batches of matrices the row-balanced small-N kernel takes,
+    which need none up to a break-even batch (20 tokens from 8192 rows on,
+    else 32; Q6_K only on rows wider than 4096 columns, up to 56): one launch
+    of up to 64 tokens where rows_tokens takes the shape, else 8 tokens per
+    launch; dense types need none, and run batches above 8 on their own GEMM
+    (nothing is launched)."""
     kern = Kernels()
 
     def pieces(cols, batch):
@@ -227,7 +229,12 @@ def test_prefill_dispatch_and_workspace():
     for t in (Q4_0, Q8_0, Q4_K):
         for batch in (9, 32):
             assert kern.workspace_bytes(t, 4096, 4096, batch) == 0
-            assert kern.kernel_name(t, 4096, 4096, batch) == "smalln_rows"
+            assert kern.kernel_name(t, 4096, 4096, batch) == "rows_tokens"
+        assert kern.kernel_name(t, 4096, 14336, 9) == "smalln_rows"
+        assert kern.kernel_name(t, 4096, 14336, 10) == "rows_tokens"
+        assert kern.kernel_name(t, 4097, 4096, 32) == "smalln_rows"
+        assert kern.kernel_name(t, 6144, 2048, 9) == "rows_tokens"
+        assert kern.kernel_name(t, 6145, 2048, 9) == "smalln_rows"
         assert kern.workspace_bytes(t, 4096, 4096, 33) == pieces(4096, 33)
         assert kern.workspace_bytes(t, 14336, 4096, 20) == 0
         assert kern.workspace_bytes(t, 14336, 4096, 21) == pieces(4096, 21)
@@ -235,7 +242,12 @@ def test_prefill_dispatch_and_workspace():
         assert kern.workspace_bytes(t, 4096, 4096, 512) == pieces(4096, 512)
         assert kern.kernel_name(t, 4096, 4096, 512) == "prefill_f16"
     assert kern.workspace_bytes(Q6_K, 4096, 14336, 56) == 0
-    assert kern.kernel_name(Q6_K, 4096, 14336, 56) == "smalln_rows"
+    assert kern.kernel_name(Q6_K, 4096, 14336, 9) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 4096, 14336, 56) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 4097, 14336, 16) == "smalln_rows"
+    assert kern.kernel_name(Q6_K, 8192, 14336, 16) == "smalln_rows"
+    assert kern.kernel_name(Q6_K, 8192, 14336, 17) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 8193, 14336, 17) == "prefill_mfma"
     assert kern.kernel_name(Q6_K, 4096, 14336, 57) == "prefill_mfma"
     assert kern.workspace_bytes(Q6_K, 4096, 4096, 9) == 4096 // 32 * 136 * 32
     assert kern.workspace_bytes(Q6_K, 4096, 4096, 512) == 4096 // 32 * 136 * 512
