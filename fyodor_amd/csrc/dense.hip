@@ -7,6 +7,7 @@
 #include "formats.h"
 #include "kernels.h"
 #include "fyodor_hip.h"
+#include <limits.h>
 #include <stdint.h>
 
 namespace fy {
@@ -120,6 +121,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 template <unsigned T> constexpr int kElem = T == F32 ? 4 : 2;
+// A buffer offset past every range (at most 2^31 - 1 bytes), also 16 bytes on.
+constexpr int kOutside = INT_MIN;
 template <unsigned T> constexpr int kPieces = T == F32 ? 3 : T == F16 ? 2 : 1;   // of a weight
 constexpr int kPlaneBytes = kGemmTokens * kGemmK * 2;   // one piece of a step's tokens
 
@@ -151,32 +154,37 @@ __device__ __forceinline__ void split(const float (&v)[2 * P], uint32_t (&out)[N
 
 // This lane's weights of a step as loaded: slice s (of four) holds columns
 // 16 s + 8 h .. + 7 of its row (the two lanes of a row read 32 or 64
-// consecutive bytes per slice). ALIGNED: rows 16-byte aligned, else element by
-// element. Columns past the row's end hold whatever follows (the buffer range
-// bounds it): their activations are zeros, and where a product of zero is no
-// number the output is computed again.
+// consecutive bytes per slice). ALIGN: bytes that every row's start is a
+// multiple of, 16, 4 or 2 (one load each). Columns past the row's end hold
+// whatever follows (the buffer range bounds it): their activations are zeros,
+// and where a product of zero is no number the output is computed again. Whole
+// steps past the wavefront's columns [.., kend) are read too with 16-byte loads
+// (a select per slice costs more); the narrow loads skip them, as offsets outside
+// the range.
 template <unsigned T>
 struct GemmWeights {
     u32x4 w[T == F32 ? 8 : 4];
 };
 
 // Slice s of the step at column kc.
-template <unsigned T, bool ALIGNED>
-__device__ __forceinline__ void load_slice(GemmWeights<T> &st, __amdgpu_buffer_rsrc_t wb, int cols, int row, int kc, int s)
+template <unsigned T, int ALIGN>
+__device__ __forceinline__ void load_slice(GemmWeights<T> &st, __amdgpu_buffer_rsrc_t wb, int cols, int row, int kc, int s,
+    int kend)
 {
     constexpr int kPer = T == F32 ? 2 : 1;   // 16-byte words per slice
     const int h = (int)((threadIdx.x >> 5) & 1);
-    const int at = (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)(kc + 16 * s + 8 * h)) * kElem<T>);
+    const int at = ALIGN == 16 || kc < kend
+                       ? (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)(kc + 16 * s + 8 * h)) * kElem<T>) : kOutside;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-        if constexpr (ALIGNED) {
+        if constexpr (ALIGN == 16) {
             st.w[kPer * s + q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, at + 16 * q, 0, 0));
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int off = at + 16 * q + 4 * e;
-                st.w[kPer * s + q][e] = T == F32 ? __builtin_amdgcn_raw_buffer_load_b32(wb, off, 0, 0)
-                                                 : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wb, off, 0, 0) |
+                st.w[kPer * s + q][e] = ALIGN == 4 ? __builtin_amdgcn_raw_buffer_load_b32(wb, off, 0, 0)
+                                                   : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wb, off, 0, 0) |
                                                        (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wb, off + 2, 0, 0) << 16;
             }
         }
@@ -196,14 +204,16 @@ __device__ __forceinline__ Tokens tokens_of()
     return {16 * (t >> 6) + ((t & 63) >> 4), 4 * (t & 15)};
 }
 
-template <bool ALIGNED>
-__device__ __forceinline__ void load_tokens(float (&x)[16], __amdgpu_buffer_rsrc_t xb, int cols, int t0, int kc)
+template <int ALIGN>
+__device__ __forceinline__ void load_tokens(float (&x)[16], __amdgpu_buffer_rsrc_t xb, int cols, int t0, int kc, int kend)
 {
     const Tokens t = tokens_of();
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int at = (int)(((uint32_t)(t0 + t.first + 4 * q) * (uint32_t)cols + (uint32_t)(kc + t.col)) * 4u);
-        if constexpr (ALIGNED) {
+        const int at = ALIGN == 16 || kc < kend
+                           ? (int)(((uint32_t)(t0 + t.first + 4 * q) * (uint32_t)cols + (uint32_t)(kc + t.col)) * 4u)
+                           : kOutside;
+        if constexpr (ALIGN == 16) {
             const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xb, at, 0, 0));
             x[4 * q] = v.x, x[4 * q + 1] = v.y, x[4 * q + 2] = v.z, x[4 * q + 3] = v.w;
         } else {
@@ -306,7 +316,7 @@ __device__ float plain_dot(const uint8_t *w, const float *x, int cols, int row, 
 // Workgroup (row tile, token tile, split z) covers the 64-column steps
 // [z per, (z + 1) per) of the split count gridDim.z; with one split it
 // writes Y, else its partial sums to part[z][token][row] for dense_combine.
-template <unsigned T, bool ALIGNED>
+template <unsigned T, int ALIGN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_gemm(
     const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int rows, int cols, int batch,
     int per, float *__restrict__ part)
@@ -339,7 +349,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     auto at = [&](int i) { return first + i * kGemmK; };
     auto step = [&](int i, int odd, GemmWeights<T> &cur, float (&xs)[16], float (&xn)[16]) {
         // (Past the last step nobody computes on what is requested.)
-        load_tokens<ALIGNED>(xn, xb, cols, t0, at(i + 2));
+        load_tokens<ALIGN>(xn, xb, cols, t0, at(i + 2), kend);
         __builtin_amdgcn_sched_barrier(0);
         cut_tokens(xs, at(i + 1), kend);
         const uint8_t *buf = sx[ks][odd];
@@ -377,7 +387,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 mul(1, 0, 1);
             }
             if constexpr (kPieces<T> > 2) mul(1, 0, 2);
-            load_slice<T, ALIGNED>(cur, wb, cols, row, at(i + 2), s);
+            load_slice<T, ALIGN>(cur, wb, cols, row, at(i + 2), s, kend);
             constexpr int kMfma = 2 * (kPieces<T> == 1 ? 3 : kPieces<T> == 2 ? 5 : 6);
 #pragma unroll
             for (int q = 0; q < kMfma; ++q) {
@@ -390,15 +400,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __syncthreads();
     };
     if (steps) {
-        load_tokens<ALIGNED>(x0, xb, cols, t0, at(0));
+        load_tokens<ALIGN>(x0, xb, cols, t0, at(0), kend);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) load_slice<T, ALIGNED>(w0, wb, cols, row, at(0), s);
+        for (int s = 0; s < 4; ++s) load_slice<T, ALIGN>(w0, wb, cols, row, at(0), s, kend);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) load_slice<T, ALIGNED>(w1, wb, cols, row, at(1), s);
+        for (int s = 0; s < 4; ++s) load_slice<T, ALIGN>(w1, wb, cols, row, at(1), s, kend);
         cut_tokens(x0, at(0), kend);
         store_tokens(x0, 0, sx[ks][0], big);
         store_tokens(x0, 1, sx[ks][0], big);
-        load_tokens<ALIGNED>(x0, xb, cols, t0, at(1));
+        load_tokens<ALIGN>(x0, xb, cols, t0, at(1), kend);
     }
     __syncthreads();
     // Two steps per pass: the registers of one take the loads of the next
@@ -483,8 +493,10 @@ __global__ __launch_bounds__(256) void dense_combine(const float *__restrict__ p
 // (of which the largest magnitude and the rows' bits cost 3 to 5 us at 512.)
 // At 512 tokens that is 1010 (F16), 730 (BF16) and 900 (F32) TFLOP/s issued
 // of the 1406 a large bf16 product reaches here: what bounds it now. Rows of
-// a multiple of 16 bytes load 16 bytes per lane; the others element by
-// element (F32 300 x 1002, 300 tokens: 39 -> 16.5 us).
+// a multiple of 16 bytes load 16 bytes per lane, of 4 bytes 4 (F16 1000 x 1002,
+// 700 tokens: 55 with the fp32 cores, 57 in loads of 2, 30 in loads of 4), the
+// others element by element (F16 1000 x 1001 the same: 55, 60 with the steps past
+// the end loaded too, 47 without).
 template <unsigned T>
 hipError_t launch_gemm(const uint8_t *w, const float *x, float *y, int rows, int cols, int batch, int splits,
     float *part, hipStream_t s)
@@ -493,9 +505,11 @@ hipError_t launch_gemm(const uint8_t *w, const float *x, float *y, int rows, int
     const dim3 grid((unsigned)((rows + kGemmRows - 1) / kGemmRows), (unsigned)((batch + kGemmTokens - 1) / kGemmTokens),
                     (unsigned)splits);
     if ((size_t)cols * kElem<T> % 16 == 0)
-        hipLaunchKernelGGL((dense_gemm<T, true>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
-    else
-        hipLaunchKernelGGL((dense_gemm<T, false>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
+        hipLaunchKernelGGL((dense_gemm<T, 16>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
+    else if ((size_t)cols * kElem<T> % 4 == 0)
+        hipLaunchKernelGGL((dense_gemm<T, 4>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
+    else if constexpr (T != F32)
+        hipLaunchKernelGGL((dense_gemm<T, 2>), grid, dim3(512), 0, s, w, x, y, rows, cols, batch, per, part);
     if (splits > 1) {
         const size_t n = (size_t)batch * rows;
         const size_t blocks = (n + 255) / 256;

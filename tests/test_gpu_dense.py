@@ -113,7 +113,7 @@ def stored(t, v):
 # Columns about the 64-column step, its halves between the two column groups
 # (an odd number of steps, one step, a step of one column) and unaligned rows;
 # tokens and rows about their tiles of 64 and 128.
-EDGES = [(127, 8, 9), (128, 63, 64), (1, 64, 65), (129, 65, 63), (130, 136, 9), (257, 192, 130), (5, 321, 66),
+EDGES = [(127, 8, 9), (128, 63, 64), (1, 64, 65), (129, 65, 63), (130, 136, 9), (257, 192, 130), (5, 321, 66), (131, 330, 65),
          (128, 1096, 64), (128, 2184, 10)]
 
 
