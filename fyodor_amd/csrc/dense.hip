@@ -313,6 +313,144 @@ __device__ float plain_dot(const uint8_t *w, const float *x, int cols, int row, 
     return wave_sum(s);
 }
 
+// ---- the fp32 matrix cores -------------------------------------------------
+//
+// A tile of 64 tokens x 128 rows on v_mfma_f32_32x32x2_f32, by four wavefronts:
+// wavefront wr computes the 64 tokens of rows 32 wr .. 32 wr + 31 as two 32 x 32
+// tiles, each in two accumulator chains (even and odd chunks) added at the end.
+// K advances 32 columns per chunk: the tokens' 64 x 32 and the rows' 128 x 32
+// values go through LDS as fp32 (rows padded to 36 floats: conflict-free 16-byte
+// reads), the next chunk's through registers while the matrix cores work. MFMA
+// step s takes column 16 h + s in lane half h, for both operands alike.
+constexpr int kChunk = 32, kPitch = 36;
+constexpr int kChunkFloats = (kGemmRows + kGemmTokens) * kPitch;   // of LDS
+
+// Thread t (of 256): W row t / 2, columns 16 (t % 2) .. + 15; X token t / 4,
+// columns 8 (t % 4) .. + 7.
+struct Chunk {
+    float w[16], x[8];
+};
+
+// The chunk at column kc of [.., kend): zeros past it. Rows and tokens past the
+// last read zeros or stay unused (buffer ranges).
+template <unsigned T>
+__device__ __forceinline__ void load_chunk(Chunk &c, __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb, int cols,
+    int r0, int t0, int kc, int kend)
+{
+    const int t = threadIdx.x & 255;
+    const int row = r0 + (t >> 1), wcol = kc + 16 * (t & 1);
+    const int tok = t0 + (t >> 2), xcol = kc + 8 * (t & 3);
+    if ((size_t)cols * kElem<T> % 16 == 0 && kc + kChunk <= kend) {
+        const int wo = (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)wcol) * kElem<T>);
+#pragma unroll
+        for (int q = 0; q < (T == F32 ? 4 : 2); ++q) {
+            const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wb, wo + 16 * q, 0, 0));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t u = v[e];
+                if constexpr (T == F32) c.w[4 * q + e] = __builtin_bit_cast(float, u);
+                else c.w[8 * q + 2 * e] = widen<T>(u), c.w[8 * q + 2 * e + 1] = widen<T>(u >> 16);
+            }
+        }
+        const int xo = (int)(((uint32_t)tok * (uint32_t)cols + (uint32_t)xcol) * 4u);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xb, xo + 16 * q, 0, 0));
+            c.x[4 * q] = v.x, c.x[4 * q + 1] = v.y, c.x[4 * q + 2] = v.z, c.x[4 * q + 3] = v.w;
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int k = wcol + e;
+        const int off = k < kend ? (int)(((uint32_t)row * (uint32_t)cols + (uint32_t)k) * kElem<T>) : kOutside;
+        if constexpr (T == F32) c.w[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wb, off, 0, 0));
+        else c.w[e] = widen<T>(__builtin_amdgcn_raw_buffer_load_b16(wb, off, 0, 0));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int k = xcol + e;
+        const int off = k < kend ? (int)(((uint32_t)tok * (uint32_t)cols + (uint32_t)k) * 4u) : kOutside;
+        c.x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xb, off, 0, 0));
+    }
+}
+
+__device__ __forceinline__ void store_chunk(const Chunk &c, float *sw)
+{
+    const int t = threadIdx.x & 255;
+    float *w = sw + (t >> 1) * kPitch + 16 * (t & 1), *x = sw + (kGemmRows + (t >> 2)) * kPitch + 8 * (t & 3);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *(float4 *)(w + 4 * q) = make_float4(c.w[4 * q], c.w[4 * q + 1], c.w[4 * q + 2], c.w[4 * q + 3]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        *(float4 *)(x + 4 * q) = make_float4(c.x[4 * q], c.x[4 * q + 1], c.x[4 * q + 2], c.x[4 * q + 3]);
+}
+
+// The tile's sums over `chunks` chunks of columns [k0, kend), in sw (kChunkFloats
+// of LDS of these four wavefronts). Every wavefront of the workgroup calls it with
+// the same number of chunks: it meets them at barriers.
+template <unsigned T>
+__device__ __forceinline__ void fp32_tile(f32x16 (&acc)[2][2], __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb,
+    int cols, int r0, int t0, int k0, int kend, int chunks, int wr, float *sw)
+{
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+    Chunk c;
+    load_chunk<T>(c, wb, xb, cols, r0, t0, k0, kend);
+    auto step = [&](int i, int chain) {
+        __syncthreads();   // the operand reads of the chunk before are done
+        store_chunk(c, sw);
+        __syncthreads();
+        if (i + 1 < chunks) load_chunk<T>(c, wb, xb, cols, r0, t0, k0 + kChunk * (i + 1), kend);
+        const float *pw = sw + (32 * wr + (lane & 31)) * kPitch + 16 * h;
+        const float *px = sw + (kGemmRows + (lane & 31)) * kPitch + 16 * h;
+        float b[16], a0[16], a1[16];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 w = *(const float4 *)(pw + 4 * q), v0 = *(const float4 *)(px + 4 * q),
+                         v1 = *(const float4 *)(px + 32 * kPitch + 4 * q);
+            b[4 * q] = w.x, b[4 * q + 1] = w.y, b[4 * q + 2] = w.z, b[4 * q + 3] = w.w;
+            a0[4 * q] = v0.x, a0[4 * q + 1] = v0.y, a0[4 * q + 2] = v0.z, a0[4 * q + 3] = v0.w;
+            a1[4 * q] = v1.x, a1[4 * q + 1] = v1.y, a1[4 * q + 2] = v1.z, a1[4 * q + 3] = v1.w;
+        }
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            acc[0][chain] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b[s], acc[0][chain], 0, 0, 0);
+            acc[1][chain] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b[s], acc[1][chain], 0, 0, 0);
+        }
+    };
+    int i = 0;
+    for (; i + 1 < chunks; i += 2) step(i, 0), step(i + 1, 1);
+    if (i < chunks) step(i, 0);
+}
+
+// Short rows: four wavefronts and 27 KiB of LDS per tile, several workgroups on a
+// CU, where the kernel above spends most of its one workgroup's time on filling
+// its pipeline and on meeting. launch_dense_gemm says where the line lies.
+template <unsigned T>
+__global__ __launch_bounds__(256) void dense_gemm(const uint8_t *__restrict__ w, const float *__restrict__ x,
+    float *__restrict__ y, int rows, int cols, int batch)
+{
+    __shared__ __align__(16) float sw[kChunkFloats];
+    const int lane = threadIdx.x & 63, h = lane >> 5, wr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = blockIdx.x * kGemmRows, t0 = blockIdx.y * kGemmTokens;
+    const __amdgpu_buffer_rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(w), (short)0, (int)((size_t)rows * cols * kElem<T>), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(x), (short)0, (int)((size_t)batch * cols * 4), 0x00020000);
+    f32x16 acc[2][2] = {};
+    fp32_tile<T>(acc, wb, xb, cols, r0, t0, 0, cols, (cols + kChunk - 1) / kChunk, wr, sw);
+    // D[token][row]: register i of lane l holds token 8 (i / 4) + 4 h + i % 4 of
+    // its 32, row l % 32.
+    const int row = r0 + 32 * wr + (lane & 31);
+    if (row >= rows) return;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const int token = t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3);
+        if (token < batch) y[(size_t)token * rows + row] = acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15];
+    }
+}
+
 // Workgroup (row tile, token tile, split z) covers the 64-column steps
 // [z per, (z + 1) per) of the split count gridDim.z; with one split it
 // writes Y, else its partial sums to part[z][token][row] for dense_combine.
@@ -550,6 +688,26 @@ bool dense_gemm_supported(unsigned type, int rows, int cols, int batch)
            (size_t)batch * rows <= (size_t)INT32_MAX;
 }
 
+// Rows short enough for the fp32 matrix cores (no column splits there). us, bf16 /
+// fp32 cores, 4096 rows by 333 and 2048 tokens (192 and 1024 tiles):
+//   columns   64             128            160            192            256            320
+//   F16     10.0/6.7      9.9/9.0       12.2/10.4      12.5/11.9      12.6/14.9      15.0/17.7
+//           35.7/18.5    35.5/27.1      44.0/32.4      45.5/38.3      45.7/47.9      55.4/56.9
+//   F32     11.9/6.6     12.3/8.3       15.8/9.6       15.8/11.1      15.8/13.7      18.7/16.4
+//           43.0/19.3    44.6/27.5      57.4/33.5      57.5/38.5      58.1/48.8      71.5/61.2
+// (F32, 384: 18.7/18.7 and 73.5/70.3; BF16 as F16). Rows that are not multiples of
+// 16 bytes, whose loads the fp32 tile does one by one: F16 66 columns 9.7/10.4 and
+// 34.4/28.4, 98 9.7/13.6 and 34.3/37.8; 155 (2-byte loads on both sides) 18.1/16.7
+// and 66.2/44.0, 193 20.1/21.3 and 74.3/57.8; F32 82 11.0/10.3 and 39.3/29.1, 155
+// 14.2/15.9 and 51.9/43.8.
+static bool dense_gemm_short(unsigned type, int rows, int cols, int batch)
+{
+    const long tiles = (long)((rows + kGemmRows - 1) / kGemmRows) * ((batch + kGemmTokens - 1) / kGemmTokens);
+    const bool many = tiles > 256;   // more than one workgroup per CU
+    if (type == F32) return cols <= (cols % 4 == 0 ? (many ? 448 : 320) : many ? 160 : 88);
+    return cols <= (cols % 8 == 0 ? (many ? 192 : 160) : cols % 2 == 0 ? (many ? 80 : 64) : many ? 224 : 160);
+}
+
 hipError_t launch_dense_gemm(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
     int batch, void *workspace, size_t workspace_bytes, hipStream_t s)
 {
@@ -559,6 +717,13 @@ hipError_t launch_dense_gemm(unsigned type, const uint8_t *w, const float *x, fl
     const size_t need = dense_gemm_workspace(rows, cols, batch);
     const int splits = need && workspace && workspace_bytes >= need ? dense_gemm_splits(rows, cols, batch) : 1;
     float *part = (float *)workspace;
+    if (dense_gemm_short(type, rows, cols, batch)) {
+        const dim3 grid((unsigned)((rows + kGemmRows - 1) / kGemmRows), (unsigned)((batch + kGemmTokens - 1) / kGemmTokens));
+        if (type == F32) hipLaunchKernelGGL(dense_gemm<F32>, grid, dim3(256), 0, s, w, x, y, rows, cols, batch);
+        else if (type == F16) hipLaunchKernelGGL(dense_gemm<F16>, grid, dim3(256), 0, s, w, x, y, rows, cols, batch);
+        else hipLaunchKernelGGL(dense_gemm<BF16>, grid, dim3(256), 0, s, w, x, y, rows, cols, batch);
+        return hipGetLastError();
+    }
     if (type == F32) return launch_gemm<F32>(w, x, y, rows, cols, batch, splits, part, s);
     if (type == F16) return launch_gemm<F16>(w, x, y, rows, cols, batch, splits, part, s);
     return launch_gemm<BF16>(w, x, y, rows, cols, batch, splits, part, s);

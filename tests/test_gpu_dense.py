@@ -114,7 +114,11 @@ def stored(t, v):
 # (an odd number of steps, one step, a step of one column) and unaligned rows;
 # tokens and rows about their tiles of 64 and 128.
 EDGES = [(127, 8, 9), (128, 63, 64), (1, 64, 65), (129, 65, 63), (130, 136, 9), (257, 192, 130), (5, 321, 66), (131, 330, 65),
-         (128, 1096, 64), (128, 2184, 10)]
+         (128, 1096, 64), (128, 2184, 10),
+         # Short rows on the fp32 cores: their 32-column chunks, the longest that
+         # take them in one and in several workgroups per CU, and the next ones.
+         (70, 31, 66), (129, 32, 70), (65, 33, 65), (127, 96, 100), (130, 160, 64), (130, 161, 64), (66, 168, 65),
+         (140, 320, 40), (140, 324, 40), (4100, 192, 520), (4100, 200, 520), (2100, 448, 1000)]
 
 
 @pytest.mark.parametrize("t", [F32, F16, BF16], ids=lambda t: TYPE_NAMES[t])
