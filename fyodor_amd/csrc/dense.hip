@@ -7,6 +7,7 @@
 #include "formats.h"
 #include "kernels.h"
 #include "fyodor_hip.h"
+#include <float.h>
 #include <limits.h>
 #include <stdint.h>
 
@@ -102,7 +103,8 @@ hipError_t launch_type(const uint8_t *w, const float *x, float *y, int rows, int
 // to about 2^-125 (|w| + |x|), and a non-finite value, or one that rounds to
 // infinity, leaves NaN or infinity in its outputs. Outputs small enough for the
 // first to show (against the largest operand that the workgroup met) or not
-// finite are computed again as plain fp32 dots.
+// finite are computed again as plain fp32 dots, or with their tile on the fp32
+// matrix cores, unless what their operands hold says that they stand.
 //
 // Work split. A workgroup of eight wavefronts owns 64 tokens x 128 rows;
 // wavefront (wr, ks) computes the 64 tokens of rows 32 wr .. 32 wr + 31 over
@@ -335,9 +337,8 @@ struct Chunk {
 // last read zeros or stay unused (buffer ranges).
 template <unsigned T>
 __device__ __forceinline__ void load_chunk(Chunk &c, __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb, int cols,
-    int r0, int t0, int kc, int kend)
+    int r0, int t0, int kc, int kend, int t)
 {
-    const int t = threadIdx.x & 255;
     const int row = r0 + (t >> 1), wcol = kc + 16 * (t & 1);
     const int tok = t0 + (t >> 2), xcol = kc + 8 * (t & 3);
     if ((size_t)cols * kElem<T> % 16 == 0 && kc + kChunk <= kend) {
@@ -375,9 +376,8 @@ __device__ __forceinline__ void load_chunk(Chunk &c, __amdgpu_buffer_rsrc_t wb, 
     }
 }
 
-__device__ __forceinline__ void store_chunk(const Chunk &c, float *sw)
+__device__ __forceinline__ void store_chunk(const Chunk &c, float *sw, int t)
 {
-    const int t = threadIdx.x & 255;
     float *w = sw + (t >> 1) * kPitch + 16 * (t & 1), *x = sw + (kGemmRows + (t >> 2)) * kPitch + 8 * (t & 3);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -394,14 +394,17 @@ template <unsigned T>
 __device__ __forceinline__ void fp32_tile(f32x16 (&acc)[2][2], __amdgpu_buffer_rsrc_t wb, __amdgpu_buffer_rsrc_t xb,
     int cols, int r0, int t0, int k0, int kend, int chunks, int wr, float *sw)
 {
-    const int lane = threadIdx.x & 63, h = lane >> 5;
+    // Opaque: a caller's registers hold none of this before it gets here.
+    int t = threadIdx.x & 255;
+    asm("" : "+v"(t));
+    const int lane = t & 63, h = lane >> 5;
     Chunk c;
-    load_chunk<T>(c, wb, xb, cols, r0, t0, k0, kend);
+    load_chunk<T>(c, wb, xb, cols, r0, t0, k0, kend, t);
     auto step = [&](int i, int chain) {
         __syncthreads();   // the operand reads of the chunk before are done
-        store_chunk(c, sw);
+        store_chunk(c, sw, t);
         __syncthreads();
-        if (i + 1 < chunks) load_chunk<T>(c, wb, xb, cols, r0, t0, k0 + kChunk * (i + 1), kend);
+        if (i + 1 < chunks) load_chunk<T>(c, wb, xb, cols, r0, t0, k0 + kChunk * (i + 1), kend, t);
         const float *pw = sw + (32 * wr + (lane & 31)) * kPitch + 16 * h;
         const float *px = sw + (kGemmRows + (lane & 31)) * kPitch + 16 * h;
         float b[16], a0[16], a1[16];
@@ -449,6 +452,85 @@ __global__ __launch_bounds__(256) void dense_gemm(const uint8_t *__restrict__ w,
         const int token = t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3);
         if (token < batch) y[(size_t)token * rows + row] = acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15];
     }
+}
+
+// ---- outputs that the pieces may have missed ---------------------------------
+//
+// Flagged outputs of a wavefront that are computed again one by one (about 3 us
+// each over 4096 columns) before their operands are looked at (25 us for 64
+// tokens), and that are afterwards, before the whole tile runs again (210 us).
+// us, 4096 x 4096 F16 by 333 tokens, 80 without: every token NaN 107, one token with
+// an infinity 210, three 308, all 314 (the fp32 cores alone: 220 whatever the
+// input; every flagged output as a dot: 4100 to 4600), one of 1e30 114, half the
+// products zero by disjoint columns 94 (1250), a diagonal matrix 101 (2130).
+constexpr int kFew = 8, kMany = 64;
+
+struct Review {
+    int votes[3][4];          // [round][row group]: outputs left
+    uint32_t rows[3][4];      // their rows
+    uint32_t tokens[4][2];    // [row group][lane half]: of the first round, bit i as output i of a lane
+    uint2 token[64], row[128];
+};
+
+// The bits of the largest magnitude among columns [k0, k1) of the row at `at`, and
+// of the least that is not zero, minus 1 (all ones: every one is zero). By the
+// wavefront.
+template <unsigned T>
+__device__ uint2 range_of(const uint8_t *v, size_t at, int k0, int k1)
+{
+    uint32_t most = 0, least = ~0u;
+#pragma unroll 16
+    for (int k = k0 + (int)(threadIdx.x & 63); k < k1; k += 64) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, weight_at<T>(v, at + k)) & 0x7FFFFFFFu;
+        most = most > b ? most : b;
+        least = least < b - 1 ? least : b - 1;
+    }
+    for (int o = 32; o; o >>= 1) {
+        const uint32_t m = (uint32_t)__shfl_xor((int)most, o, 64), l = (uint32_t)__shfl_xor((int)least, o, 64);
+        most = most > m ? most : m;
+        least = least < l ? least : l;
+    }
+    return make_uint2(most, least);
+}
+
+// Whether output v of a token and a row of these ranges is what plain sums give:
+// not a number because an operand is none; or finite (so no operand was infinite
+// or rounded to infinity), and zero for want of operands, or of operands whose
+// pieces and products are all above the subnormals, or large against what
+// subnormals of this token and row can have lost.
+__device__ __forceinline__ bool stands(uint2 t, uint2 w, float v, float cols)
+{
+    if (t.x > 0x7F800000u || w.x > 0x7F800000u) return true;
+    if (!(__builtin_fabsf(v) <= FLT_MAX)) return false;
+    if (t.y == ~0u || w.y == ~0u) return true;
+    const float tm = __builtin_bit_cast(float, t.y + 1), wm = __builtin_bit_cast(float, w.y + 1);
+    if (tm >= 0x1p-100f && wm >= 0x1p-100f && tm * wm >= 0x1p-98f) return true;
+    return __builtin_fabsf(v) >=
+           cols * 0x1p-99f * __builtin_fmaxf(__builtin_bit_cast(float, t.x), __builtin_bit_cast(float, w.x));
+}
+
+// Shares out what is left of the four row groups in this round; the most that one
+// of them has, the same in every wavefront.
+__device__ __forceinline__ int review_votes(Review &rv, uint32_t again, int wr, int ks, int round)
+{
+    if (ks == 0) {
+        const uint64_t lanes = __ballot(again != 0);
+        int n = __popc(again);
+        uint32_t m = again;
+        for (int o = 1; o < 64; o *= 2) {
+            n += __shfl_xor(n, o, 64);
+            if (o < 32) m |= (uint32_t)__shfl_xor((int)m, o, 64);
+        }
+        if ((threadIdx.x & 31) == 0) {
+            if (round == 0) rv.tokens[wr][(threadIdx.x >> 5) & 1] = m;
+            rv.votes[round][wr] = n;
+            rv.rows[round][wr] = (uint32_t)lanes | (uint32_t)(lanes >> 32);
+        }
+    }
+    __syncthreads();
+    int most = 0;
+    for (int i = 0; i < 4; ++i) most = most > rv.votes[round][i] ? most : rv.votes[round][i];
+    return __builtin_amdgcn_readfirstlane(most);
 }
 
 // Workgroup (row tile, token tile, split z) covers the 64-column steps
@@ -556,12 +638,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         step(i + 1, 1, w1, x1, x0);
     }
     if (steps & 1) step(steps - 1, 0, w0, x0, x1);
+    // (Formed anew: nothing of it lives in registers through the loop.)
+    int end_lane = threadIdx.x & 63;
+    asm("" : "+v"(end_lane));
+    const int end_h = end_lane >> 5, end_row = r0 + 32 * wr + (end_lane & 31);
     // The halves meet in LDS. D[token][row]: register i of lane l holds token
     // 8 (i / 4) + 4 h + i % 4 of its token tile, row l % 32.
-    float *meet = (float *)&sx[0][0][0] + 2048 * wr + lane, *most = (float *)&sx[0][0][0] + 8192;
-    uint32_t *bits = (uint32_t *)most + 8 + 64 * wr + lane;
+    float *meet = (float *)&sx[0][0][0] + 2048 * wr + end_lane, *most = (float *)&sx[0][0][0] + 8192;
+    uint32_t *bits = (uint32_t *)most + 8 + 64 * wr + end_lane;
     for (int o = 32; o; o >>= 1) big = __builtin_fmaxf(big, __shfl_xor(big, o, 64));
-    if (lane == 0) most[wave] = big;
+    if (end_lane == 0) most[wave] = big;
     if (ks == 1) {
         *bits = seen;
 #pragma unroll
@@ -570,44 +656,93 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             for (int i = 0; i < 16; ++i) meet[64 * (16 * t + i)] = acc[t][0][i] + acc[t][1][i];
     }
     __syncthreads();
-    if (ks == 1) return;
-    for (int i = 0; i < 8; ++i) big = __builtin_fmaxf(big, most[i]);
-    // cols 2^-125 2 big is lost at most; it may weigh 2^-25.
-    const float least = (float)cols * 0x1p-99f * big;
+    // Outputs to look at again, by output i of the lane (its row, 32 tokens).
+    uint32_t again = 0;
     float *out = gridDim.z == 1 ? y : part + (size_t)blockIdx.z * batch * rows;
-    auto token = [&](int i) { return t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * h + (i & 3); };
-    uint32_t again = 0, zero = 0;
+    auto token = [&](int i) { return t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * end_h + (i & 3); };
+    if (ks == 0) {
+        for (int i = 0; i < 8; ++i) big = __builtin_fmaxf(big, most[i]);
+        // cols 2^-125 2 big is lost at most; it may weigh 2^-25.
+        const float least = (float)cols * 0x1p-99f * big;
+        uint32_t zero = 0;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const float v = (acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15]) + meet[64 * i];
-        if (row < rows && token(i) < batch) {
-            const float m = __builtin_fabsf(v);
-            if (!(m >= least && m <= 3.402823466e38f)) again |= 1u << i;
-            if (m == 0.f) zero |= 1u << i;
-            out[(size_t)token(i) * rows + row] = v;
-        }
-    }
-    if (__ballot(again != 0) == 0) return;
-    // The zeros of a row of zeros stand.
-    seen |= *bits;
-    seen |= (uint32_t)__shfl_xor((int)seen, 32, 64);
-    if ((seen & (T == F32 ? 0x7FFFFFFFu : 0x7FFF7FFFu)) == 0) again &= ~zero;
-    for (int i = 0; i < 32; ++i)
-        for (int half = 0; half < 2; ++half) {
-            uint64_t need = __ballot(again >> i & 1) & 0xFFFFFFFFull << 32 * half;
-            if (need == 0) continue;
-            const int tok = __builtin_amdgcn_readlane(token(i), 32 * half);
-            // So do those of a token of zeros.
-            bool any = false;
-#pragma unroll 16
-            for (int k = k0 + lane; k < k1; k += 64) any |= x[(size_t)tok * cols + k] != 0.f;
-            if (__ballot(any) == 0) need &= ~__ballot(zero >> i & 1);
-            while (need) {
-                const int l = __ffsll((unsigned long long)need) - 1, at = __builtin_amdgcn_readlane(row, l);
-                need &= need - 1;
-                const float v = plain_dot<T>(w, x, cols, at, tok, k0, k1);
-                if (lane == l) out[(size_t)tok * rows + at] = v;
+        for (int i = 0; i < 32; ++i) {
+            const float v = (acc[i >> 4][0][i & 15] + acc[i >> 4][1][i & 15]) + meet[64 * i];
+            if (end_row < rows && token(i) < batch) {
+                const float m = __builtin_fabsf(v);
+                if (!(m >= least && m <= FLT_MAX)) again |= 1u << i;
+                if (m == 0.f) zero |= 1u << i;
+                out[(size_t)token(i) * rows + end_row] = v;
             }
+        }
+        // The zeros of a row of zeros stand.
+        seen |= *bits;
+        seen |= (uint32_t)__shfl_xor((int)seen, 32, 64);
+        if ((seen & (T == F32 ? 0x7FFFFFFFu : 0x7FFF7FFFu)) == 0) again &= ~zero;
+    }
+    // Few of them: plain dots. More: what their tokens hold settles most, then
+    // what their rows hold; of what is left, few are dots again, else the tile is
+    // computed again on the fp32 matrix cores.
+    Review &rv = *(Review *)((float *)&sx[0][0][0] + 8192 + 8 + 256);
+    int left = review_votes(rv, again, wr, ks, 0);
+    if (left == 0) return;
+    for (int stage = 0; stage < 2 && left > kFew; ++stage) {
+        int n = 0;   // the stage's tokens or rows, dealt to the eight wavefronts
+        if (stage == 0) {
+            for (int f = 0; f < 2; ++f) {
+                uint32_t m = rv.tokens[0][f] | rv.tokens[1][f] | rv.tokens[2][f] | rv.tokens[3][f];
+                for (m = __builtin_amdgcn_readfirstlane(m); m; m &= m - 1) {
+                    const int i = __ffs(m) - 1, at = t0 + 32 * (i >> 4) + 8 * ((i >> 2) & 3) + 4 * f + (i & 3);
+                    if ((n++ & 7) != wave) continue;
+                    const uint2 r = range_of<F32>((const uint8_t *)x, (size_t)at * cols, k0, k1);
+                    if (end_lane == 0) rv.token[32 * f + i] = r;
+                }
+            }
+        } else {
+            for (int f = 0; f < 4; ++f)
+                for (uint32_t m = __builtin_amdgcn_readfirstlane(rv.rows[1][f]); m; m &= m - 1) {
+                    const int i = __ffs(m) - 1;
+                    if ((n++ & 7) != wave) continue;
+                    const uint2 r = range_of<T>(w, (size_t)(r0 + 32 * f + i) * cols, k0, k1);
+                    if (end_lane == 0) rv.row[32 * f + i] = r;
+                }
+        }
+        __syncthreads();
+        // Before the rows are looked at: anything, but that F16 is in its range.
+        const uint2 any = T == F16 ? make_uint2(0x477FE000u, 0x33800000u - 1) : make_uint2(0x7F7FFFFFu, 0u);
+        uint32_t keep = again;
+        for (uint32_t m = again; m; m &= m - 1) {
+            const int i = __ffs(m) - 1;
+            const float v = out[(size_t)token(i) * rows + end_row];
+            if (stands(rv.token[32 * end_h + i], stage ? rv.row[32 * wr + (end_lane & 31)] : any, v, (float)cols)) keep &= ~(1u << i);
+        }
+        again = keep;
+        left = review_votes(rv, again, wr, ks, stage + 1);
+    }
+    if (left > kMany) {
+        f32x16 sum[2][2] = {};
+        static_assert(2 * kChunkFloats * 4 <= (int)sizeof(sx), "both halves' chunks");
+        fp32_tile<T>(sum, wb, xb, cols, r0, t0, first, kend, 2 * steps, wr, (float *)&sx[0][0][0] + ks * kChunkFloats);
+        __syncthreads();
+        if (ks == 1) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) meet[64 * i] = sum[i >> 4][0][i & 15] + sum[i >> 4][1][i & 15];
+        }
+        __syncthreads();
+        if (ks == 1) return;
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            if (end_row < rows && token(i) < batch)
+                out[(size_t)token(i) * rows + end_row] = (sum[i >> 4][0][i & 15] + sum[i >> 4][1][i & 15]) + meet[64 * i];
+        return;
+    }
+    if (ks == 1) return;
+    for (int i = 0; i < 32; ++i)
+        for (uint64_t need = __ballot(again >> i & 1); need; need &= need - 1) {
+            const int l = __ffsll((unsigned long long)need) - 1;
+            const int at = __builtin_amdgcn_readlane(end_row, l), tok = __builtin_amdgcn_readlane(token(i), l);
+            const float v = plain_dot<T>(w, x, cols, at, tok, k0, k1);
+            if (end_lane == l) out[(size_t)tok * rows + at] = v;
         }
 }
 

@@ -167,3 +167,58 @@ def test_dense_gemm_non_finite(hip, t):
         finite = np.isfinite(exact)
         assert np.array_equal(y[~finite & ~np.isnan(exact)], exact[~finite & ~np.isnan(exact)])
         assert np.all(np.abs(y[finite] - exact[finite]) <= (cols / 16 + 16) * 2.0 ** -24 * m[finite])
+
+
+@pytest.mark.parametrize("t", [F32, F16, BF16], ids=lambda t: TYPE_NAMES[t])
+@pytest.mark.parametrize("kind", ["nan-tokens", "nan-rows", "inf-token", "inf-tokens", "inf-rows", "huge", "masked", "padded",
+                                  "tiny", "tiny-rows"])
+def test_dense_gemm_reviewed_tiles(hip, t, kind):
+    """Inputs of which a tile has more outputs to look at again than are
+    computed one by one: whether they stand is told from their tokens' and
+    rows' ranges, the rest come one by one or with their whole tile on the fp32
+    cores. Infinities and NaN as plain sums give them, the other outputs to the
+    bound of test_dense_gemm_pieces."""
+    for rows, cols, batch in [(200, 704, 130), (130, 901, 65)]:
+        rng = np.random.default_rng(rows + cols + t)
+        wv = rng.uniform(-1, 1, (rows, cols)).astype(np.float32)
+        x = rng.uniform(-1, 1, (batch, cols)).astype(np.float32)
+        if kind == "nan-tokens":
+            x[rng.random(batch) < 0.5, 7] = np.nan
+        elif kind == "nan-rows":
+            wv[rng.random(rows) < 0.5, 9] = np.nan
+        elif kind == "inf-token":
+            x[40, [3, 650]] = np.inf, 1.0
+        elif kind == "inf-tokens":
+            x[rng.random(batch) < 0.6, 11], x[::9, 12] = np.inf, -np.inf
+        elif kind == "inf-rows":
+            wv[rng.random(rows) < 0.3, 600], x[5::7, 600] = -np.inf, 0.0
+        elif kind == "huge":
+            x[3::16] *= np.float32(2.0 ** 120)
+            x[50, 100] = np.float32(3.4028e38)
+            wv[:, 100] = np.abs(wv[:, 100]) * np.float32(0.125)
+        elif kind == "masked":
+            x[rng.random(batch) < 0.5, :400] = 0.0
+            wv[rng.random(rows) < 0.7, 400:] = 0.0
+            x[::5] = np.where(rng.random((len(x[::5]), cols)) < 0.98, 0.0, x[::5])
+        elif kind == "padded":
+            x[50:], wv[120:] = 0.0, 0.0
+        elif kind == "tiny":
+            x[1::2] *= np.float32(2.0 ** -118)
+            x[::11, 400:] = np.float32(2.0 ** -130)
+        else:
+            wv[1::3] *= np.float32(2.0 ** (-14 if t == F16 else -110))
+            x[::3] *= np.float32(2.0 ** -20)
+            wv[::4, 300:] = 0.0
+        w, wv = stored(t, wv)
+        with np.errstate(invalid="ignore", over="ignore"):
+            exact = np.stack([np.sum(wv.astype(np.float64) * x[b].astype(np.float64), axis=1) for b in range(batch)])
+            m = np.stack([np.sum(np.abs(wv.astype(np.float64) * x[b].astype(np.float64)), axis=1) for b in range(batch)])
+        finite = np.isfinite(exact) & (np.abs(exact) < 2.0 ** 127)
+        for workspace in (True, False):
+            print(f"{TYPE_NAMES[t]} {kind} {rows}x{cols} batch {batch} workspace {workspace}", flush=True)
+            y = run(hip, w, t, x, rows, cols, batch, workspace).astype(np.float64)
+            assert np.array_equal(np.isnan(y), np.isnan(exact))
+            assert np.array_equal(y[np.isinf(exact)], exact[np.isinf(exact)])
+            assert np.all(y[m == 0] == 0)
+            # (2^-149: an output's own last place.)
+            assert np.all(np.abs(y[finite] - exact[finite]) <= (cols / 16 + 16) * 2.0 ** -24 * m[finite] + 2.0 ** -149)
