@@ -395,18 +395,36 @@ hipError_t launch_tile(const float *q, int q_stride, const float *keys, const fl
 }  // namespace
 
 // The runs this kernel takes from the per-head kernel, which fills the chip
-// with one workgroup per (token, head) and so wins on few of them: its time
-// grows with tokens x heads, this kernel's stays that of one workgroup until
-// the chip is full. Measured per-head / this kernel, us (MI355X): 32 heads of
-// 128, 64 tokens: 128 positions 17.0 / 17.0, 512 46.5 / 37.8, 4096 368 / 226;
-// 48 tokens: 36.4 / 37.0 at 512. 32 of 64, 64 tokens: 128 positions
-// 13.7 / 10.5, 512 26.8 / 22.3; 48 tokens 21.4 / 22.2 at 512. 16 heads of 256
-// (two key tiles per step, one wavefront per SIMD): 256 tokens 129 / 126 at
-// 512 positions, 1703 / 861 at 4096; 128 tokens 77 / 125 and 682 / 867.
-bool attention_tile_supported(int count, int heads, int kv_heads, int width)
+// with one workgroup per (token, head) and so wins on few of them and on short
+// ranges: its time grows with tokens x heads x range, this kernel's stays that of
+// one workgroup's key steps (17 us with one, 7.6 more for each, at width 128) until
+// the chip is full. The positions are on the device: what is known of the ranges
+// is that none exceeds max_length or the window. us, per-head / this kernel:
+//   tokens x heads     window 64      128        512     run's end 512   4096
+//    64 x 32 of 128    12.3/17.1  15.3/24.6   44.4/45.0   42.7/36.8    340/221
+//    96 x 32 of 128    16.5/17.2  20.9/24.8   63.2/45.2   64.5/43.9    502/222
+//   128 x 32 of 128    20.5/17.4  27.1/25.1   82.5/45.3   86.0/44.0    657/221
+//    64 x 32 of  64     9.2/10.5  10.0/14.7   25.7/26.5   24.8/22.2    172/140
+//   256 x 16 of 256    25.5/47.3  43.1/60.3    148/140     119/125    1653/862
+//   512 x 16 of 256    48.0/48.3  81.0/61.2    289/141     166/126    3395/872
+//   200 x 48 of 256    58.0/92.6  99.0/119     402/285     441/269    9108/1700
+// and of runs from position 0: 64, 96 and 128 x 32 of 128 12.7/17.3, 17.1/17.2,
+// 22.7/17.4; of 64 8.9/10.3, 11.8/10.4, 14.9/10.4; 256 and 512 x 16 of 256 48/72,
+// 166/126; 512 x 8 of 256 79/125; 200 x 48 of 256 94/78. So, in (token, head)
+// pairs, at width 64 and 128: 4096, 3072 unless a window below 512 keeps the ranges
+// short, 2048 where they may reach 512 (a window 1024); at width 256: 24576, 8192
+// unless a window is below 256, 4096 where they may reach 512 in a run that may
+// reach 1024. Fewer pairs that see little of a longer cache lose what the
+// figures show; a caller that knows its run's end passes it as max_length.
+bool attention_tile_supported(int count, int heads, int kv_heads, int width, int max_length, int window)
 {
     if (width != 64 && width != 128 && width != 256) return false;
-    if ((long)count * heads < (width <= 128 ? 2048 : 4096)) return false;
+    const bool windowed = window > 0 && window < max_length;
+    const int range = windowed ? window : max_length;
+    const long pairs = (long)count * heads;
+    if (width <= 128 ? pairs < (windowed && range < 512 ? 4096 : range < (windowed ? 1024 : 512) ? 3072 : 2048)
+                     : pairs < (windowed && range < 256 ? 24576 : range < 512 || max_length < 1024 ? 8192 : 4096))
+        return false;
     const long rows = (long)count * (heads / kv_heads);
     // 32-bit row counts, grid and per-tile buffer offsets.
     return rows <= (long)1 << 30 && (rows / 32 + 1) * kv_heads <= (long)1 << 30 &&

@@ -183,7 +183,7 @@ hipError_t launch_attention_split(const float *q, int q_stride, const float *key
 // Runs of prompt tokens on the fp32 matrix cores (attention_tile.hip): width
 // 64, 128 or 256, q, keys, values and out 16-byte aligned, q_stride a multiple
 // of 4; no scores scratch at any length. launch_attention chooses it.
-bool attention_tile_supported(int count, int heads, int kv_heads, int width);
+bool attention_tile_supported(int count, int heads, int kv_heads, int width, int max_length, int window);
 hipError_t launch_attention_tile(const float *q, int q_stride, const float *keys, const float *values, float *out,
     const int *positions, int count, int heads, int kv_heads, int width, int max_length, int window, float scale,
     hipStream_t s);

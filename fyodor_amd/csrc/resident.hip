@@ -1165,7 +1165,7 @@ hipError_t launch_attention(const float *q, int q_stride, const float *keys, con
     if (width > kMaxWidth) return hipErrorInvalidValue;
     const bool aligned = (q_stride & 3) == 0 &&
                          (((uintptr_t)q | (uintptr_t)keys | (uintptr_t)values | (uintptr_t)out) & 15u) == 0;
-    if (aligned && attention_tile_supported(count, heads, kv_heads, width))
+    if (aligned && attention_tile_supported(count, heads, kv_heads, width, max_length, window))
         return launch_attention_tile(q, q_stride, keys, values, out, positions, count, heads, kv_heads, width,
                                      max_length, window, scale, s);
     const dim3 grid((unsigned)heads, (unsigned)count);

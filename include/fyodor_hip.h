@@ -229,7 +229,9 @@ NYA_HIP_EXPORT int nya_hip_rope_qkv(uintptr_t q, size_t q_stride, uintptr_t k, s
  * (at most max_length) of keys / values ([max_length][kv_heads * width]
  * rows), a softmax, and out[i] = sum_t p_t v_t (backend/core/llm_cpu.c:491-511).
  * window > 0 keeps the last `window` of those positions, as the engine
- * bounds a sliding layer's attention (:486-488); 0 keeps all. `scores` is
+ * bounds a sliding layer's attention (:486-488); 0 keeps all. A max_length that
+ * is no longer than the run reaches lets short runs take the kernel that is
+ * faster on them. `scores` is
  * scratch of count * heads * max_length floats, needed (and used) only
  * when max_length exceeds 8192. */
 NYA_HIP_EXPORT int nya_hip_attention(uintptr_t q, size_t q_stride, uintptr_t keys, uintptr_t values, uintptr_t out,

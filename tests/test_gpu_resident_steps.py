@@ -347,6 +347,12 @@ RUN_CASES = [  # heads, kv_heads, width, max_length, count, first, window: count
     (32, 8, 128, 300, 64, 0, 0), (32, 8, 128, 700, 70, 601, 0), (32, 4, 64, 129, 65, 64, 0), (24, 8, 128, 250, 100, 33, 0),
     (32, 32, 128, 97, 97, 0, 40), (32, 1, 64, 200, 64, 130, 0), (32, 8, 128, 600, 513, 40, 64), (16, 8, 256, 300, 257, 17, 0),
     (16, 8, 256, 400, 256, 140, 100), (8, 2, 128, 8300, 257, 8000, 0), (64, 8, 256, 600, 512, 80, 0),
+    # The same edges past the thresholds of short ranges and windows, and at both sides of them.
+    (32, 8, 128, 400, 160, 0, 0), (32, 4, 64, 300, 131, 64, 0), (24, 8, 128, 350, 180, 33, 0), (32, 32, 128, 140, 140, 0, 40),
+    (32, 1, 64, 300, 140, 130, 0), (32, 8, 128, 512, 64, 440, 0), (32, 8, 128, 511, 64, 440, 0), (32, 8, 128, 511, 96, 300, 0),
+    (32, 4, 64, 1200, 70, 1100, 1024), (32, 4, 64, 700, 96, 600, 512), (32, 4, 64, 700, 95, 600, 512),
+    (16, 8, 256, 1024, 257, 750, 0), (16, 8, 256, 600, 513, 17, 256), (48, 8, 256, 600, 515, 40, 100),
+    (16, 8, 256, 1023, 300, 700, 0), (48, 8, 256, 200, 171, 0, 0), (16, 8, 256, 1100, 260, 800, 512),
     # Width 64 about the last grid of one row tile per workgroup, odd and even tile counts.
     (32, 4, 64, 600, 512, 20, 0), (32, 4, 64, 560, 513, 20, 0), (16, 16, 64, 400, 300, 0, 0), (32, 8, 64, 300, 250, 9, 0)]
 
