@@ -579,8 +579,9 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
     // over the groups, us before and now: 14336 x 4096 x24 31.6, 28.1; 4096 x
     // 4096 x64 28.5, 26.1; 4096 x 14336 x40 92.7, 77.9; 2048 x 2048 x512 22.0,
     // 21.8. With more workgroups than CUs two of the single kind share one
-    // (2560 x 2048 x512 28.9, 33.2 split; 6144 x 4096 x256 49.7, 58.6).
-    const bool split = (long)(tiles + 3) / 4 * whole1 <= 256;
+    // (2560 x 2048 x512 28.9, 33.2 split; 6144 x 4096 x256 49.7, 58.6). One group
+    // leaves the second set nothing (5917 x 256 x40: 8.0, 9.7 split).
+    const bool split = cols > kGroupCols && (long)(tiles + 3) / 4 * whole1 <= 256;
     const dim3 grid2((unsigned)((tiles + 7) / 8 * tb2));
     const dim3 grid((unsigned)((tiles + (wide ? 7 : 3)) / (wide ? 8 : 4) * tb));
 #define FY_PREFILL(TT, RTT, TWW, KSS, G, TB) \
