@@ -112,13 +112,13 @@ hipError_t launch_prefill(unsigned type, const uint8_t *w, const float *x, float
     int whole, void *workspace, hipStream_t stream);
 const char *prefill_kernel(unsigned type);
 
-// Whole 256-column groups (prefill_tile.hip): every Q8_0, Q4_0 and Q6_K batch
-// of them, Q4_K batches that fill the chip. np: the tokens the workspace holds
+// Whole 256-column groups (prefill_tile.hip): every Q6_K batch of them, Q8_0 and
+// Q4_0 but for some of up to eight groups, Q4_K batches that fill the chip. np: the tokens the workspace holds
 // pieces of (batch rounded up to a multiple of 32).
 bool prefill_tile_supported(unsigned type, int rows, int cols, int whole);
 hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
     int whole, void *workspace, int np, hipStream_t s);
-// The other Q4_K batches, and Q8_0 / Q4_0 rows with a short last group
+// The other batches, and Q8_0 / Q4_0 rows with a short last group
 // (prefill_f16.hip).
 size_t prefill_f16_workspace(int cols, int batch);
 hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,

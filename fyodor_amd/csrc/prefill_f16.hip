@@ -1,8 +1,8 @@
 // Prefill GEMM Y[m][row] = sum_k W[row][k] * X[m][k] for batches above 8 on
 // gfx950 fp16 MFMA (v_mfma_f32_32x32x16_f16): Q4_K batches too small to fill
-// the chip with the 256 x 64 workgroups of prefill_tile.hip, and Q8_0 / Q4_0
-// rows whose last 256-column group is short. Also splits the activations for
-// both files.
+// the chip with the 256 x 64 workgroups of prefill_tile.hip, Q8_0 / Q4_0 rows
+// whose last 256-column group is short, and short Q8_0 / Q4_0 rows where that
+// file's rule says so. Also splits the activations for both files.
 //
 // Numbers. The weights enter the MFMA as exact fp16 integers: Q4_K sc * q
 // (<= 63 * 15 = 945), Q8_0 q, Q4_0 q - 8. Each token's activations are scaled
@@ -568,7 +568,7 @@ hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, f
     const int tiles = (rows + kTileRows - 1) / kTileRows;
     // Two token tiles per wavefront (each weight operand serves four MFMAs)
     // where one workgroup per CU of 256 rows x 64 tokens fills the chip (Q4_K
-    // batches that do are prefill_tile.hip's).
+    // batches that need more than one for some CU are prefill_tile.hip's).
     const int tb2 = (batch + 2 * kTokens - 1) / (2 * kTokens), whole2 = (whole + 2 * kTokens - 1) / (2 * kTokens);
     const int tb = (batch + kTokens - 1) / kTokens, whole1 = (whole + kTokens - 1) / kTokens;
     const bool pair = (long)(tiles + 7) / 8 * whole2 >= 256;

@@ -19,11 +19,12 @@
 // matrix cores busy 65 % of the cycles at a clock that has fallen to 1.67 GHz
 // (1107 issued TFLOP/s; a library fp16 product reaches 1495).
 //
-// Wide workgroups: four wavefronts, 256 rows x 64 tokens. The accumulators
-// (128 registers with a K-quant's running group) leave two wavefronts per
-// SIMD: two workgroups per CU, each other's cover at the barriers. K advances
-// 128 columns per step; copies for the next step go out at a step's start.
-// Narrow workgroups split the columns four ways (below).
+// Wide workgroups: four wavefronts, 256 rows x 64 tokens (Q8_0 and Q4_0 also x
+// 32, where that evens the CUs out). The accumulators (128 registers with a
+// K-quant's running group) leave two wavefronts per SIMD: two workgroups per CU,
+// each other's cover at the barriers. K advances 128 columns per step; copies
+// for the next step go out at a step's start. Narrow workgroups split the
+// columns four ways (below).
 //
 // The pieces go global -> LDS directly (buffer_load ... lds). 16-byte chunk c
 // of token t lies at place c ^ (t % 16) of the token's 256 bytes (the
@@ -644,15 +645,15 @@ __device__ __forceinline__ void narrow_gemm(const uint8_t *w, const Pieces &p, f
     store_tile<T, TT>(st, tile_of, p, y, rows, batch, np, m0);
 }
 
-// Wide: 256 rows x 64 tokens, 64 KiB of step buffers, two workgroups per CU.
+// Wide: 256 rows x 32 TT tokens, 32 TT KiB of step buffers, two workgroups per CU.
 // Narrow: 64 WR rows x 32 TT tokens, 128 KiB, one workgroup per CU.
-template <unsigned T>
+template <unsigned T, int TT>
 __device__ __forceinline__ void wide_kernel(const uint8_t *w, const Pieces &p, float *__restrict__ y, int rows, int cols,
     int batch, int np, int token_blocks)
 {
-    __shared__ __align__(16) uint8_t s0[32768], s1[32768];
-    __shared__ __align__(16) uint8_t sums[T == Q4_K ? 2 * kSumTile : 16];
-    wide_gemm<T, 2>(w, p, y, rows, cols, batch, np, token_blocks, (lds_u8 *)s0, (lds_u8 *)s1, (lds_u8 *)sums);
+    __shared__ __align__(16) uint8_t s0[16384 * TT], s1[16384 * TT];
+    __shared__ __align__(16) uint8_t sums[T == Q4_K ? TT * kSumTile : 16];
+    wide_gemm<T, TT>(w, p, y, rows, cols, batch, np, token_blocks, (lds_u8 *)s0, (lds_u8 *)s1, (lds_u8 *)sums);
 }
 
 template <unsigned T, int TT, int WR>
@@ -676,7 +677,7 @@ template <unsigned T, int TT, int WR>
 __global__ __launch_bounds__(WR == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(WR == 1 ? 1 : 2, WR == 1 ? 1 : 2))) void prefill_f16(
     const uint8_t *w, Pieces p, float *__restrict__ y, int rows, int cols, int batch, int np, int token_blocks)
 {
-    if constexpr (WR == 0) wide_kernel<T>(w, p, y, rows, cols, batch, np, token_blocks);
+    if constexpr (WR == 0) wide_kernel<T, TT>(w, p, y, rows, cols, batch, np, token_blocks);
     else narrow_kernel<T, TT, WR>(w, p, y, rows, cols, batch, np, token_blocks);
 }
 
@@ -684,7 +685,7 @@ template <int TT, int WR>
 __global__ __launch_bounds__(WR == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(WR == 1 ? 1 : 2, WR == 1 ? 1 : 2))) void prefill_mfma(
     const uint8_t *w, Pieces p, float *__restrict__ y, int rows, int cols, int batch, int np, int token_blocks)
 {
-    if constexpr (WR == 0) wide_kernel<Q6_K>(w, p, y, rows, cols, batch, np, token_blocks);
+    if constexpr (WR == 0) wide_kernel<Q6_K, TT>(w, p, y, rows, cols, batch, np, token_blocks);
     else narrow_kernel<Q6_K, TT, WR>(w, p, y, rows, cols, batch, np, token_blocks);
 }
 
@@ -714,6 +715,18 @@ hipError_t launch_wide(unsigned type, const uint8_t *w, const Pieces &p, float *
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
+
+// 256 rows x 32 tokens (Q8_0 and Q4_0).
+hipError_t launch_half(unsigned type, const uint8_t *w, const Pieces &p, float *y, int rows, int cols, int batch, int np,
+    hipStream_t s)
+{
+    const int token_blocks = (batch + 31) / 32, per = 4 * kTileRows * kR;
+    const dim3 grid((unsigned)(((long)rows + per - 1) / per * token_blocks)), block(256);
+    if (type == Q8_0) hipLaunchKernelGGL((prefill_f16<Q8_0, 1, 0>), grid, block, 0, s, FY_ARGS);
+    else if (type == Q4_0) hipLaunchKernelGGL((prefill_f16<Q4_0, 1, 0>), grid, block, 0, s, FY_ARGS);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
 #undef FY_ARGS
 
 }  // namespace
@@ -722,37 +735,76 @@ hipError_t launch_wide(unsigned type, const uint8_t *w, const Pieces &p, float *
 // workgroups (one per CU) of 64 rows x 32 tokens, then 128 x 32, then 128 x 64;
 // past that 256 x 64 wide. Q4_K's narrow shapes close a group (its minimums
 // and scales) every 64 columns of a wavefront and lose to the 32-token
-// workgroups of prefill_f16.hip, which keep every batch too small to fill the
-// chip wide. Measured, us (64x32 / 128x32 / 128x64 / 256x64; the int8 kernel
-// before for Q6_K, prefill_f16.hip for the others):
+// workgroups of prefill_f16.hip, which keep every batch that would not give some
+// CU two of 256 x 64 (with just one for each, the older form of that shape is
+// faster: 8192 x 4096 x512 76.8 us there, 84.3 here; 4096 x 4096 x1024 79.4, 85.3).
+// Measured, us (64x32 / 128x32 / 128x64 / 256x64; the int8 kernel before for Q6_K,
+// prefill_f16.hip for the others):
 //   Q6_K 4096x14336 x128     82 / 105 / 136 / 249   218
 //   Q6_K 4096x14336 x256    148 / 115 / 140 / 251   275
 //   Q6_K 4096x14336 x512    288 / 220 / 171 / 256   502
 //   Q6_K 4096x4096  x512    102 /  74 /  62 /  83   161
-//   Q8_0 4096x4096  x64      23 /  27 /  42 /  69    39
-//   Q8_0 11008x4096 x256    122 /  92 / 104 /  84    92
-//   Q8_0 11008x4096 x512    213 / 167 / 154 / 124   158
-//   Q4_0 4096x11008 x64      45 /  54 /  93 / 165    85
-//   Q4_0 4096x11008 x512    185 / 134 / 124 / 188   141
 //   Q4_K 14336x4096 x512    331 / 220 / 218 / 123   136
 //   Q4_K 11264x2048 x256     88 /  60 /  73 /  41    42
 //   Q4_K 4096x4096  x512    105 /  69 /  65 /  70    48
-enum Shape { kRows64, kRows128, kRows128Wide, kRows256, kElsewhere };
+// Tall Q6_K matrices are bound by their weights on few tokens: 128256 x 4096, 9
+// tokens 157 (the int8 kernel's 16-token workgroups: 182).
+//
+// Q8_0 and Q4_0: where that shape leaves its last round of the CUs nearly empty,
+// 256 x 32, or for rows of up to eight groups prefill_f16.hip (128 x 32, two to
+// a CU, no shares to add), if its time by the model below is less. us: the kernels
+// before this file's, the shape by the workgroups alone, now:
+//   Q8_0 42240x5632 x22    70 /  98 / 60     Q4_0 16896x14336 x89   154 / 227 / 138
+//   Q8_0 7126x8192 x283   114 / 155 / 96     Q4_0 7872x256 x182      12 /  18 /  11
+//   Q8_0 6432x512 x305     17 /  21 / 16     Q4_0 992x1024 x994      18 /  20 /  17
+enum Shape { kRows64, kRows128, kRows128Wide, kRows256, kRows256Half, kElsewhere };
 
-static Shape shape_of(unsigned type, int rows, int whole)
+// A shape's time in 10 ns, for Q8_0 (Q4_0's are the same to a few percent):
+// `pair` and `single` per 256-column group of two workgroups on a CU and of one
+// (narrow ones come one at a time), `round` per such workgroup, `once`, and
+// per 1000 tokens and group, and 1000 tokens, the split. Fitted to 1600 shapes
+// (256 to 80000 rows, 256 to 14336 columns, 21 to 2048 tokens): half of the times
+// within 4 %, nine of ten within 12; what the rule takes is within 2 % of the
+// faster of both kernels before it on all but 12 of them, 0.5 to 4 us off there.
+struct ShapeTime {
+    long pair, single, round, once, split_group, split;
+};
+constexpr ShapeTime kTimes[] = {{172, 86, 405, 419, 57, 229},  {228, 114, 638, 207, 41, 239},
+                                {418, 209, 1273, 0, 24, 645},  {680, 413, 278, 613, 35, 214},
+                                {400, 240, 174, 546, 37, 193}, {256, 188, 138, 497, 30, 174}};
+
+static long time_of(Shape shape, long workgroups, long groups, long tokens)
+{
+    const ShapeTime &t = kTimes[shape];
+    const long k = (workgroups + 255) / 256;   // of the fullest CU
+    return (k / 2 * t.pair + k % 2 * t.single) * groups + k * t.round + t.once +
+           tokens * (groups * t.split_group + t.split) / 1000;
+}
+
+static Shape shape_of(unsigned type, int rows, int cols, int whole)
 {
     const long t32 = ((long)whole + 31) / 32, t64 = ((long)whole + 63) / 64;
     auto blocks = [&](int per) { return ((long)rows + per - 1) / per; };
     if (type == Q4_K) return blocks(256) * t64 > 256 ? kRows256 : kElsewhere;
-    if (blocks(64) * t32 <= 256) return kRows64;
-    if (blocks(128) * t32 <= 256) return kRows128;
-    if (blocks(128) * t64 <= 256) return kRows128Wide;
-    return kRows256;
+    const long workgroups[] = {blocks(64) * t32,  blocks(128) * t32, blocks(128) * t64,
+                               blocks(256) * t64, blocks(256) * t32, blocks(128) * t32};
+    int shape = kRows64;
+    while (shape < kRows256 && workgroups[shape] > 256) ++shape;
+    if (type == Q6_K) return (Shape)shape;
+    const long groups = cols / kGroupCols;
+    long least = time_of((Shape)shape, workgroups[shape], groups, whole);
+    // (From 256 workgroups of 256 x 64 on, prefill_f16.hip has another shape.)
+    const int last = groups <= 8 && workgroups[kRows256] < 256 ? kElsewhere : kRows256Half;
+    for (int s = kRows256Half; s <= last; ++s) {
+        const long time = time_of((Shape)s, workgroups[s], groups, whole);
+        if (time < least) least = time, shape = s;
+    }
+    return (Shape)shape;
 }
 
 bool prefill_tile_supported(unsigned type, int rows, int cols, int whole)
 {
-    return cols % kGroupCols == 0 && shape_of(type, rows, whole) != kElsewhere;
+    return cols % kGroupCols == 0 && shape_of(type, rows, cols, whole) != kElsewhere;
 }
 
 hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols, int batch,
@@ -761,10 +813,11 @@ hipError_t launch_prefill_tile(unsigned type, const uint8_t *w, const float *x, 
     const Pieces p = pieces_of(workspace, cols, np);
     const hipError_t e = launch_split_x(x, batch, cols, p, true, s);
     if (e != hipSuccess) return e;
-    switch (shape_of(type, rows, whole)) {
+    switch (shape_of(type, rows, cols, whole)) {
     case kRows64: return launch_blocks<1, 1>(type, w, p, y, rows, cols, batch, np, s);
     case kRows128: return launch_blocks<1, 2>(type, w, p, y, rows, cols, batch, np, s);
     case kRows128Wide: return launch_blocks<2, 2>(type, w, p, y, rows, cols, batch, np, s);
+    case kRows256Half: return launch_half(type, w, p, y, rows, cols, batch, np, s);
     case kRows256: return launch_wide(type, w, p, y, rows, cols, batch, np, s);
     default: return hipErrorInvalidValue;
     }

@@ -63,9 +63,12 @@ def test_batch_and_row_tails(compute, oracle, type_id, batch):
 # One shape per workgroup form of the whole-group GEMM, with ragged rows and
 # tokens and group counts around the four-step rotation of the narrow forms and
 # the two sets of wavefronts that take every other group (Q4_K, small grids)
-# (rows, cols, batch): 64 x 32, 128 x 32, 128 x 64, 256 x 64.
+# (rows, cols, batch): 64 x 32, 128 x 32, 128 x 64, 256 x 64, and for Q8_0 and
+# Q4_0 256 x 32 (both parities of groups, ragged last token tile) and the short
+# rows that leave that file.
 TILE_FORMS = [(200, 256, 33), (75, 512, 40), (300, 768, 65), (33, 1280, 97), (2081, 1024, 513), (4097, 512, 161),
-              (4000, 1280, 129), (8161, 256, 200), (8161, 768, 200), (16100, 512, 300), (33001, 256, 170)]
+              (4000, 1280, 129), (8161, 256, 200), (8161, 768, 200), (16100, 512, 300), (33001, 256, 170),
+              (17820, 2304, 33), (33001, 768, 29), (10792, 2304, 178), (250, 2304, 40), (63, 512, 143), (3340, 768, 132)]
 
 
 @pytest.mark.parametrize("type_id", QUANT, ids=lambda t: TYPE_NAMES[t])
