@@ -399,19 +399,30 @@ hipError_t launch_type(const uint8_t *w, const float *x, float *y, int rows, int
 
 // Up to 4096 rows: a workgroup per CU. Beyond, where a CU reads x several times
 // over, 8-token launches win (Q4_K 14336 x 4096, 16 tokens: 20 us, 30 here; 6144
-// x 4096: 13.8, 15.9; Q8_0 5120 x 4096: 13.6, 18.4), but on short rows (Q4_0
-// 6144 x 2048: 12.0, 9.8) and for Q6_K, whose 8-token launches decode longest,
-// from 17 tokens on (8192 x 14336: 16 tokens 55, 54 here; 33 tokens 133, 104;
-// 6144 x 8192: 33 tokens 77, 57). Nine tokens of wide rows are one launch of
-// eight and a matvec there (Q4_K 4096 x 14336: 25.3, 26.4 here).
+// x 4096: 13.8, 15.9; Q8_0 5120 x 4096: 13.6, 18.4) but on short rows, and on
+// those of up to 2048 columns from 25 tokens on, a launch more. us, 8-token
+// launches / here, 5632 rows by 9, 16, 24 and 28 tokens:
+//   Q4_K  1024 columns   7.0/6.0   7.7/6.1  11.5/10.3  14.7/10.3
+//         1536           7.4/8.8   8.9/9.0  13.2/14.8  16.8/14.8
+//         2048           7.9/9.4   9.4/9.6  14.1/15.8  17.7/15.8
+//   Q4_0  1024           6.5/5.9   7.1/6.0  10.7/10.3  13.6/10.3
+//   Q8_0   512           7.0/5.7   7.1/5.7  10.5/9.6   13.4/9.5
+//         1024 (6144)    6.4/7.1   7.3/7.1  10.9/11.2  14.0/11.2
+// Q6_K, whose 8-token launches decode longest, from 17 tokens on (8192 x 14336: 16
+// tokens 55, 54 here; 33 tokens 133, 104; 6144 x 8192: 33 tokens 77, 57), but for
+// three whole launches of the tallest (8192 x 14336, 24 tokens 81.5, 86; 8192 x
+// 4608 32.9, 33.9; 6144 x 8192 51.5, 49.1). Nine tokens of wide rows are one
+// launch of eight and a matvec up to 4096 rows (Q4_K 4096 x 14336: 25.3, 26.4 here).
 bool rows_tokens_supported(unsigned type, int rows, int cols, int batch)
 {
     if (type != Q4_K && type != Q4_0 && type != Q8_0 && type != Q6_K) return false;
     if (rows <= 0 || cols <= 0 || cols % kGroupCols || batch <= 8 || batch > kRowsTokens) return false;
     // x within a 32-bit buffer range.
     if ((size_t)kRowsTokens * cols * 4 > (size_t)INT32_MAX) return false;
-    if (type == Q6_K) return rows <= 4096 || (rows <= 8192 && batch > 16);
-    return rows <= 4096 ? batch > 9 || cols <= 4096 : rows <= 6144 && cols <= 2048;
+    if (type == Q6_K)
+        return rows <= 4096 || (rows <= 8192 && batch > 16 && (rows <= 6144 || batch <= 20 || batch > 24));
+    if (rows <= 4096) return batch > 9 || cols <= 4096;
+    return rows <= 6144 && cols <= (batch > 24 ? 2048 : type == Q8_0 ? 512 : 1024);
 }
 
 hipError_t launch_rows_tokens(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,

@@ -233,8 +233,16 @@ def test_prefill_dispatch_and_workspace():
         assert kern.kernel_name(t, 4096, 14336, 9) == "smalln_rows"
         assert kern.kernel_name(t, 4096, 14336, 10) == "rows_tokens"
         assert kern.kernel_name(t, 4097, 4096, 32) == "smalln_rows"
-        assert kern.kernel_name(t, 6144, 2048, 9) == "rows_tokens"
-        assert kern.kernel_name(t, 6145, 2048, 9) == "smalln_rows"
+        # Between 4097 and 6144 rows: short rows, longer ones from 25 tokens on.
+        short = 512 if t == Q8_0 else 1024
+        assert kern.kernel_name(t, 6144, short, 9) == "rows_tokens"
+        assert kern.kernel_name(t, 6145, short, 9) == "smalln_rows"
+        for batch in (9, 16, 24):
+            assert kern.kernel_name(t, 5632, short + 256, batch) == "smalln_rows"
+            assert kern.kernel_name(t, 5632, 2048, batch) == "smalln_rows"
+        assert kern.kernel_name(t, 6144, 2048, 25) == "rows_tokens"
+        assert kern.kernel_name(t, 6144, 2304, 25) == "smalln_rows"
+        assert kern.kernel_name(t, 6145, 2048, 25) == "smalln_rows"
         assert kern.workspace_bytes(t, 4096, 4096, 33) == pieces(4096, 33)
         assert kern.workspace_bytes(t, 14336, 4096, 20) == 0
         assert kern.workspace_bytes(t, 14336, 4096, 21) == pieces(4096, 21)
@@ -247,6 +255,11 @@ def test_prefill_dispatch_and_workspace():
     assert kern.kernel_name(Q6_K, 4097, 14336, 16) == "smalln_rows"
     assert kern.kernel_name(Q6_K, 8192, 14336, 16) == "smalln_rows"
     assert kern.kernel_name(Q6_K, 8192, 14336, 17) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 6144, 14336, 24) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 6145, 14336, 20) == "rows_tokens"
+    assert kern.kernel_name(Q6_K, 6145, 14336, 21) == "smalln_rows"
+    assert kern.kernel_name(Q6_K, 6145, 14336, 24) == "smalln_rows"
+    assert kern.kernel_name(Q6_K, 8192, 14336, 25) == "rows_tokens"
     assert kern.kernel_name(Q6_K, 8193, 14336, 17) == "prefill_mfma"
     assert kern.kernel_name(Q6_K, 4096, 14336, 57) == "prefill_mfma"
     assert kern.workspace_bytes(Q6_K, 4096, 4096, 9) == 4096 // 32 * 136 * 32
