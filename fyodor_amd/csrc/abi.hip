@@ -41,11 +41,16 @@ bool storage_bytes(unsigned type, size_t rows, size_t cols, size_t *bytes)
 // Batches above the small-N kernels' 8 columns go to the prefill GEMM (every
 // block format), except small batches of matrices the row-balanced small-N
 // kernel takes, which need no workspace and run on rows_tokens.hip or, 8
-// tokens per launch, on that kernel, up to a batch measured per shape (MI355X,
-// 50 calls over rotating weights, GEMM / 8-token launches): Q4_K 14336 x 4096
-// at 16 tokens 32.0 / 22.3 us, at 24 32.6 / 33.0; Q4_K and Q8_0 4096 x 4096 at
-// 32 31.4 / 26.2 and 40.7 / 25.6 (14.4 and 15.5 on rows_tokens.hip). The Q6_K
-// output head (128256 x 4096) keeps the GEMM from 9 tokens on (173 / 198 us).
+// tokens per launch, on that kernel, up to a batch per shape. The limits are
+// older than rows_tokens.hip and than the GEMM's present forms. MI355X, us over
+// rotating weights, GEMM / without a workspace: Q4_K 14336 x 4096, 21 tokens
+// 26.7 / 30.4 (20: 30.3); Q8_0 25.8 / 38.0; Q4_K 4096 x 4096, 33 tokens 25.5 / 15.8,
+// 64 25.6 / 22.7; Q8_0 22.3 / 16.5, 22.9 / 23.0; Q6_K 4096 x 14336, 57 tokens
+// 75.5 / 71.2; Q6_K 128256 x 4096 (an output head), 9 tokens 163 / 191, 33 tokens
+// 181 / 573. They are on the slower side for 33 to about 60 tokens of up to 4096
+// rows, for Q6_K of up to 4096 rows and columns below 65 tokens (4096 x 4096, 9
+// tokens 25.7 / 9.7, 64 27.7 / 23.0), and for Q6_K of 4097 to 8192 wide rows from
+// about 33 tokens on (8192 x 14336: 33 tokens 97 without, 57 83.5 / 131).
 bool use_prefill(unsigned type, size_t rows, size_t cols, size_t batch)
 {
     if (batch <= 8 || !(type == Q4_K || type == Q6_K || type == Q8_0 || type == Q4_0)) return false;

@@ -760,7 +760,7 @@ __global__ __launch_bounds__(256) void dense_combine(const float *__restrict__ p
 // us before (one fp32 MFMA chain, 64 x 64 tiles) and now, 4096 x 4096 by
 // tokens, alone on the stream:
 //          16          333          512          2048
-//   F16    38 -> 19    219 -> 70    235 -> 85    690 -> 345
+//   F16    38 -> 19    219 -> 73    235 -> 85    690 -> 345
 //   BF16   38 -> 18    243 -> 68    241 -> 71
 //   F32    34 -> 28    208 -> 105   213 -> 115
 // (of which the largest magnitude and the rows' bits cost 3 to 5 us at 512.)

@@ -124,7 +124,8 @@ size_t prefill_f16_workspace(int cols, int batch);
 hipError_t launch_prefill_f16(unsigned type, const uint8_t *w, const float *x, float *y, int rows, int cols,
     int batch, int whole, void *workspace, hipStream_t stream);
 
-// Dense F32 / F16 / BF16 batches above 8 as one GEMM on the fp32 matrix cores
+// Dense F32 / F16 / BF16 batches above 8 as one GEMM, on the bf16 matrix cores in
+// exact pieces, short rows on the fp32 ones
 // (dense.hip).
 // Batches of matrices with few row tiles split the columns over several
 // workgroups; their partial sums need dense_gemm_workspace bytes.

@@ -31,9 +31,11 @@
 //                                          27    30    33    45    53    61    75
 //   Q4_K 4096 x 4096                       12    14          26
 //                                           9.9   9.8        14.4
-// What bounds it now: from 32 tokens on the fp32 matrix cores (60 % busy at 48
-// tokens; one wavefront's decoding and waits are covered by one other) and the
-// return path of x, which every workgroup reads whole; below that latency.
+// The tokens past the whole tiles as FMAs, Q6_K 4096 x 14336: 17 tokens 31.5, 20
+// 35.4, 24 (two tiles) 39.7; 33 46.0, 36 53.2, 48 59.6; 49 61.7, 52 68.1, 64 73.5.
+// What bounds it now: from 32 tokens on the fp32 matrix cores (61 % busy at 48
+// tokens, 48 % at 33; one wavefront's decoding and waits are covered by one other)
+// and the return path of x, which every workgroup reads whole; below that latency.
 #include "blockdot.h"
 #include "kernels.h"
 #include <limits.h>

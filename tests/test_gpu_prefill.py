@@ -1,5 +1,4 @@
-"""The prefill GEMM (batches above 8): fp16 MFMA for Q4_0 / Q8_0 / Q4_K,
-int8 MFMA for Q6_K.
+"""The prefill GEMM (batches above 8) on fp16 MFMA.
 
 - prefill shapes of the 8B-class projections at batch 128..512: sampled
   tokens (both tile edges included) against the double-precision oracle
@@ -8,8 +7,8 @@ int8 MFMA for Q6_K.
 - batch and row tails (batch 9, 127..129, 257; 200 rows = one full and one
   partial weight tile) with canaries on both sides of the output;
 - through the kernel library's C ABI: the GEMM (workspace given) against the
-  same request run through the small-N path (int8 activation digits; both
-  represent x to about 2^-22 and differ in fp32 summation order), and the
+  same request run without a workspace (fp32 activations up to 64 tokens per
+  launch, or int8 digits; the GEMM represents x to about 2^-22), and the
   workspace size it asks for.
 """
 import numpy as np
@@ -106,7 +105,7 @@ def test_prefill_matches_tiled_path(hip, type_id):
     x = synth.activations(batch, cols, 78 + type_id)
     need = kern.workspace_bytes(type_id, rows, cols, batch)
     if type_id == Q6_K:
-        assert need == cols // 32 * 136 * 64      # digits, batch rounded up to 32 tokens
+        assert need == cols // 32 * 136 * 64      # room for 136 bytes per 32 columns, batch rounded up to 32 tokens
         assert kern.kernel_name(type_id, rows, cols, batch) == "prefill_mfma"
     else:
         assert need == 64 * (4 * cols + cols // 32 * 4 + 4)   # fp16 pieces of 64 tokens
@@ -122,18 +121,19 @@ def test_prefill_matches_tiled_path(hip, type_id):
         kern.matmul(wdev, type_id, rows, cols, xdev, ydev, batch, 0, 0, stream)
         rt.sync(stream)
         tiled = rt.download(ydev, np.empty((batch, rows), dtype=np.float32))
-        # A workspace one byte short is refused by the prefill GEMM: tiled again.
+        # A workspace one byte short is refused by the prefill GEMM: the same again.
         kern.matmul(wdev, type_id, rows, cols, xdev, ydev, batch, work, need - 1, stream)
         rt.sync(stream)
         short = rt.download(ydev, np.empty((batch, rows), dtype=np.float32))
     finally:
         for p in (wdev, xdev, ydev, work):
             rt.free(p)
-    # Without the GEMM's workspace the batch runs 8 tokens at a time: on the
-    # row-balanced small-N kernel where it takes the shape (no workspace
-    # either way); else without a workspace token by token, on the batch-1
-    # matvec where the type has one (its own rounding) or on the same small-N
-    # kernel as the batches of 8 the short workspace gets.
+    # Without the GEMM's workspace the batch runs in one launch of rows_tokens
+    # where that takes it, else 8 tokens at a time: on the row-balanced small-N
+    # kernel where it takes the shape (no workspace either way); else without a
+    # workspace token by token, on the batch-1 matvec where the type has one (its
+    # own rounding) or on the same small-N kernel as the batches of 8 the short
+    # workspace gets.
     if kern.kernel_name(type_id, rows, cols, 8) == "smalln_rows" or kern.kernel_name(type_id, rows, cols, 1) == "smalln_mfma":
         assert np.array_equal(short, tiled)
     else:
