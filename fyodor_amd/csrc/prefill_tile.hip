@@ -754,9 +754,9 @@ hipError_t launch_half(unsigned type, const uint8_t *w, const Pieces &p, float *
 // 256 x 32, or for rows of up to eight groups prefill_f16.hip (128 x 32, two to
 // a CU, no shares to add), if its time by the model below is less. us: the kernels
 // before this file's, the shape by the workgroups alone, now:
-//   Q8_0 42240x5632 x22    70 /  98 / 60     Q4_0 16896x14336 x89   154 / 227 / 138
-//   Q8_0 7126x8192 x283   114 / 155 / 96     Q4_0 7872x256 x182      12 /  18 /  11
-//   Q8_0 6432x512 x305     17 /  21 / 16     Q4_0 992x1024 x994      18 /  20 /  17
+//   Q8_0 42240x5632 x22    80 / 107 /  66    Q4_0 16896x14336 x89   152 / 217 / 138
+//   Q8_0 7104x8192 x283   112 / 156 / 100    Q4_0 7872x256 x182      12 /  17 /  11
+//   Q8_0 6432x512 x305     18 /  21 /  17    Q4_0 992x1024 x994      18 /  20 /  16
 enum Shape { kRows64, kRows128, kRows128Wide, kRows256, kRows256Half, kElsewhere };
 
 // A shape's time in 10 ns, for Q8_0 (Q4_0's are the same to a few percent):
