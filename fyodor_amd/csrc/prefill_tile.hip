@@ -763,9 +763,9 @@ enum Shape { kRows64, kRows128, kRows128Wide, kRows256, kRows256Half, kElsewhere
 // `pair` and `single` per 256-column group of two workgroups on a CU and of one
 // (narrow ones come one at a time), `round` per such workgroup, `once`, and
 // per 1000 tokens and group, and 1000 tokens, the split. Fitted to 1600 shapes
-// (256 to 80000 rows, 256 to 14336 columns, 21 to 2048 tokens): half of the times
-// within 4 %, nine of ten within 12; what the rule takes is within 2 % of the
-// faster of both kernels before it on all but 12 of them, 0.5 to 4 us off there.
+// (256 to 80000 rows, 256 to 14336 columns, 21 to 2048 tokens): half of a form's
+// times within 4 to 6 %, nine of ten within 9 to 13; what the rule takes is within
+// 2 % of the faster of both kernels before it on all but 12, 0.4 to 4 us off there.
 struct ShapeTime {
     long pair, single, round, once, split_group, split;
 };
